@@ -16,14 +16,15 @@ size_t ferret_moe_permute_workspace(long long num_pairs, int E);
 size_t ferret_fp8_gemm_ue8m0_workspace(int M, int N, int K);
 int ferret_moe_w13_fp8_skinny(const void* x, const float* sx, const void* w, const float* sw,
                               const int32_t* sorted_pair, const int32_t* tiles, const int32_t* ntiles,
-                              int max_tiles, int topk, int N, int K, void* out, hipStream_t st);
+                              int max_tiles, long long num_pairs, int topk, int E, int N, int K, void* out,
+                              hipStream_t st);
 int ferret_moe_w13_fp8_tiled(const void* x, const float* sx, const void* w, const float* sw,
                              const int32_t* sorted_pair, const int32_t* tiles, const int32_t* ntiles,
                              int max_tiles, int topk, int N, int K, void* out, bool f8, hipStream_t st);
 
 int ferret_moe_w2_fp8_skinny(const void* h, const float* sh, const void* w, const float* sw,
                              const int32_t* sorted_pair, const int32_t* tiles, const int32_t* ntiles,
-                             int max_tiles, int N, int K, void* out, hipStream_t st);
+                             int max_tiles, long long num_pairs, int E, int N, int K, void* out, hipStream_t st);
 int ferret_moe_w2_fp8_tiled(const void* h, const float* sh, const void* w, const float* sw,
                             const int32_t* sorted_pair, const int32_t* tiles, const int32_t* ntiles,
                             int max_tiles, int N, int K, void* out, bool f8, hipStream_t st);
@@ -85,8 +86,8 @@ extern "C" int ferret_moe_w13_fp8_ex(const void* x, const float* sx, const void*
   FERRET_REQUIRE(T >= 1 && topk >= 1 && E >= 1 && max_tiles >= 0, FERRET_ERR_SHAPE);
   FERRET_REQUIRE(N % 256 == 0 && K % 128 == 0 && K >= 128 && K / 128 <= 128, FERRET_ERR_SHAPE);
   if (tile_m == 16)
-    return ferret_moe_w13_fp8_skinny(x, sx, w, sw, sorted_pair, tiles, ntiles, max_tiles, topk, N, K, out,
-                                     (hipStream_t)stream);
+    return ferret_moe_w13_fp8_skinny(x, sx, w, sw, sorted_pair, tiles, ntiles, max_tiles, (long long)T * topk,
+                                     topk, E, N, K, out, (hipStream_t)stream);
   if (tile_m == 128)
     return ferret_moe_w13_fp8_tiled(x, sx, w, sw, sorted_pair, tiles, ntiles, max_tiles, topk, N, K, out,
                                     (flags & FERRET_FP8_MMA_E4M3) != 0, (hipStream_t)stream);
@@ -110,7 +111,7 @@ extern "C" int ferret_moe_w2_fp8_ex(const void* h, const float* sh, const void* 
   FERRET_REQUIRE(P >= 1 && E >= 1 && max_tiles >= 0, FERRET_ERR_SHAPE);
   FERRET_REQUIRE(N % 128 == 0 && N >= 128 && K % 128 == 0 && K >= 128 && K / 128 <= 128, FERRET_ERR_SHAPE);
   if (tile_m == 16)
-    return ferret_moe_w2_fp8_skinny(h, sh, w, sw, sorted_pair, tiles, ntiles, max_tiles, N, K, out,
+    return ferret_moe_w2_fp8_skinny(h, sh, w, sw, sorted_pair, tiles, ntiles, max_tiles, P, E, N, K, out,
                                     (hipStream_t)stream);
   if (tile_m == 128)
     return ferret_moe_w2_fp8_tiled(h, sh, w, sw, sorted_pair, tiles, ntiles, max_tiles, N, K, out,

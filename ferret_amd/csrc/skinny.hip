@@ -66,6 +66,16 @@ static int try_stream(const SkinnyArgs& a_in, int dense_tiles, int max_tiles, hi
   // INT4 keeps at most one unit of scales ahead: ring depth <= KS.
   constexpr int D2 = (is_int4(F) && D > 2) ? 2 : D;
   constexpr int D4 = (is_int4(F) && D > 4) ? 4 : D;
+  if constexpr (F == kFP8 && (EPI == kSilu || RB == 4)) {
+    // The FP8 MoE products with several tiles per expert: two tiles per unit.
+    if (a.pair_tiles && max_tiles <= kStreamPairTiles) {
+      switch (plan.ks) {
+        case 2: return launch_stream<F, EPI, RB, NW, 2, D, 2>(a, slots, grid, st);
+        case 4: return launch_stream<F, EPI, RB, NW, 4, D, 2>(a, slots, grid, st);
+        case 7: return launch_stream<F, EPI, RB, NW, 7, D, 2>(a, slots, grid, st);
+      }
+    }
+  }
   switch (plan.ks) {
     case 2: return launch_stream<F, EPI, RB, NW, 2, D2>(a, slots, grid, st);
     case 4: return launch_stream<F, EPI, RB, NW, 4, D4>(a, slots, grid, st);
@@ -322,10 +332,15 @@ int ferret_fp8_gemm_skinny(const void* a_, const float* sa, const void* b, const
   return launch_skinny<kFP8, kStore, 1>(a, (M + 15) / 16, st);
 }
 
-// Decode-sized FP8 MoE w13 (tile_m = 16).
+// Decode-sized FP8 MoE w13 (tile_m = 16).  Two tiles per unit from an average
+// of 6 rows per expert: at 9.4 rows an even routing, with hardly a second tile
+// anywhere, takes 1140 us either way, a Zipf(1.1) one 1238 against 1413 us
+// (6.3 rows: 1054 against 1130); below, an even routing loses the 0.8 % the
+// pairing costs (4 rows: 1086 against 1078 us).
 int ferret_moe_w13_fp8_skinny(const void* x, const float* sx, const void* w, const float* sw,
                               const int32_t* sorted_pair, const int32_t* tiles, const int32_t* ntiles,
-                              int max_tiles, int topk, int N, int K, void* out, hipStream_t st) {
+                              int max_tiles, long long num_pairs, int topk, int E, int N, int K, void* out,
+                              hipStream_t st) {
   SkinnyArgs a{};
   a.w = static_cast<const uint8_t*>(w);
   a.w_scale = sw;
@@ -339,6 +354,7 @@ int ferret_moe_w13_fp8_skinny(const void* x, const float* sx, const void* w, con
   a.N = N;
   a.K = K;
   a.units_n = N / 32;
+  a.pair_tiles = num_pairs >= 6LL * E;
   if (max_tiles <= 0) return FERRET_OK;
   const int rc = try_stream<kFP8, kSilu, 2, 3, 8>(a, 0, max_tiles, st);
   if (rc != 1) return rc;
@@ -347,9 +363,11 @@ int ferret_moe_w13_fp8_skinny(const void* x, const float* sx, const void* w, con
 
 // Decode-sized FP8 MoE w2 / down projection (tile_m = 16): the A row and the
 // output row of a sorted row are both its routed pair (topk = 1 indexing).
+// Two tiles per unit from an average of 10 rows per expert (15.6 rows: 652
+// against 870 us; 9.4 rows: 650 against 634 us).
 int ferret_moe_w2_fp8_skinny(const void* h, const float* sh, const void* w, const float* sw,
                              const int32_t* sorted_pair, const int32_t* tiles, const int32_t* ntiles,
-                             int max_tiles, int N, int K, void* out, hipStream_t st) {
+                             int max_tiles, long long num_pairs, int E, int N, int K, void* out, hipStream_t st) {
   SkinnyArgs a{};
   a.w = static_cast<const uint8_t*>(w);
   a.w_scale = sw;
@@ -369,6 +387,7 @@ int ferret_moe_w2_fp8_skinny(const void* h, const float* sh, const void* w, cons
 // four blocks on 4 waves of 4 K-steps take 256 experts 593 -> 555 us and
 // 32 experts x 16 rows 82 -> 79 us.
   a.units_n = N / 16;  // units of the per-unit fallback (RB = 1); try_stream derives its own
+  a.pair_tiles = num_pairs >= 10LL * E;
   const int rc = try_stream<kFP8, kStore, 4, 3, 4>(a, 0, max_tiles, st);
   if (rc != 1) return rc;
   return launch_skinny<kFP8, kStore, 1>(a, max_tiles, st);

@@ -29,6 +29,7 @@ struct SkinnyArgs {
   int units_n;              // row units per token tile
   float* partial;           // stream kernel, bf16 dense split-K: fp32 [ksplit, M, N] (null: no split)
   int ksplit;               // number of K splits when partial != null
+  bool pair_tiles;          // grouped: prefer the stream kernel that takes two tiles of an expert per unit
 };
 
 template <int F>

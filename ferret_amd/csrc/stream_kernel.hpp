@@ -52,15 +52,15 @@ struct StreamFmt<kINT4> {
 template <>
 struct StreamFmt<kINT4T> : StreamFmt<kINT4> {};
 
-template <int F, int RB, int NW, int KS, int D>
+template <int F, int RB, int NW, int KS, int D, int TB = 1>
 struct StreamCfg {
   static constexpr int kWBytes = RB * 16 * StreamFmt<F>::kRowB;       // weights of one stage
   // FP8: + 256 B per stage for the 128 x 128 weight-block scale of each row block.
   static constexpr int kStage = kWBytes + (F == kFP8 ? 256 : 0);
   static constexpr int kLoads = RB * StreamFmt<F>::kInstr + (F == kFP8 ? 1 : 0);  // DMA ops per stage
   // Activation loads of one K-step (vector loads: FP8 two 16-B loads and the
-  // scale, bf16 / INT4 four 16-B loads).
-  static constexpr int kXLoads = F == kFP8 ? 3 : 4;
+  // scale, bf16 / INT4 four 16-B loads), for each of the TB token tiles.
+  static constexpr int kXLoads = (F == kFP8 ? 3 : 4) * TB;
   static constexpr int kRing = D * kStage;                            // per wave
   // INT4: the group scales of a unit (RB * 16 rows x this wave's KS K-steps,
   // 8 B per row and K-step) are copied once per unit as whole 16-B chunks:
@@ -74,16 +74,20 @@ struct StreamCfg {
   static constexpr int kSclLoads = is_int4(F) ? (RB * 16 * kSclCh + 63) / 64 : 0;
   static constexpr int kScl = is_int4(F) ? 2 * kSclBuf : 0;            // per wave
   static constexpr int kRed = NW * RB * kRedBlock * 4;                // one reduction buffer
-  static constexpr int kTiles = kStreamMaxTiles * 3 * 4;              // grouped tile table
+  // Grouped tile table: expert, then (first row, rows) of each of the TB tiles.
+  static constexpr int kTileInts = 1 + 2 * TB;
+  static constexpr int kTiles = kStreamMaxTiles * kTileInts * 4;
+  // TB > 1: the first table row of every group of tiles (16 bits each), and their count.
+  static constexpr int kLead = TB > 1 ? kStreamPairTiles * 2 + 16 : 0;
   // LDS layout, in this order: each wave's ring and INT4 scale buffers, the
   // two reduction buffers, the tile table (the kernel takes every offset from
   // here).
   static constexpr int kWaveBytes = kRing + kScl;
   static constexpr int kRedOff = NW * kWaveBytes;
   static constexpr int kTileOff = kRedOff + 2 * kRed;
-  static constexpr int kLds = kTileOff + kTiles;
-  static_assert(kRedOff % 16 == 0 && kTileOff % 16 == 0, "LDS regions 16-byte aligned");
-  static_assert(kTileOff + kStreamMaxTiles * 3 * (int)sizeof(int) == kLds, "the tile table ends the LDS");
+  static constexpr int kLeadOff = kTileOff + kTiles;
+  static constexpr int kLds = kLeadOff + kLead;
+  static_assert(kRedOff % 16 == 0 && kTileOff % 16 == 0 && kLeadOff % 16 == 0, "LDS regions 16-byte aligned");
   static_assert(!is_int4(F) || D <= KS, "INT4 unit scales are double-buffered: at most one unit ahead");
   static_assert(kLds <= 160 * 1024, "LDS budget");
   // Step s reads the fragments of step s + 1 before refilling, so item s + 1
@@ -92,7 +96,7 @@ struct StreamCfg {
   static_assert(D * (kLoads + kXLoads) + kSclLoads < 64, "vmcnt range");
   // First token tile's activations interleaved with its weight items: when the
   // ring prologue and the first unit's refills reach at most one unit ahead.
-  static constexpr bool kInterleave = D <= KS;
+  static constexpr bool kInterleave = D <= KS && TB == 1;
 };
 
 // Chunk slot of global 16-byte chunk c of LDS row `row` (per row width).
@@ -185,11 +189,54 @@ struct StepFrag {
   float sv[RB];
 };
 
+// Groups of up to TB consecutive rows of the tile table with one expert:
+// lead[g] = first table row of group g; returns the group count.  One wave
+// walks the table 64 rows at a time (eight chunks' experts loaded at once).
+template <int TB>
+__device__ __forceinline__ int group_tiles(const int32_t* tiles, int ntiles, int lane, uint16_t* lead) {
+  constexpr int B = 8;
+  int n = 0, carry_e = -1, carry_pos = 0;  // the last row walked: its expert, its place in that expert's run
+  for (int base0 = 0; base0 < ntiles; base0 += 64 * B) {
+    int ex[B];
+#pragma unroll
+    for (int b = 0; b < B; ++b) {
+      const int i = base0 + 64 * b + lane;
+      ex[b] = i < ntiles ? tiles[3 * i] : -1;
+    }
+#pragma unroll
+    for (int b = 0; b < B; ++b) {
+      const int base = base0 + 64 * b;
+      if (base >= ntiles) break;
+      const int up = __shfl_up(ex[b], 1);
+      const uint64_t starts = __ballot(ex[b] != (lane == 0 ? carry_e : up));
+      const uint64_t upto = starts & (~0ull >> (63 - lane));
+      const int pos = upto != 0 ? lane - (63 - __clzll((long long)upto)) : lane + carry_pos + 1;
+      const bool first = base + lane < ntiles && pos % TB == 0;
+      const uint64_t firsts = __ballot(first);
+      if (first) lead[n + __popcll(firsts & ((1ull << lane) - 1))] = (uint16_t)(base + lane);
+      n += __popcll(firsts);
+      carry_e = __builtin_amdgcn_readlane(ex[b], 63);
+      carry_pos = __builtin_amdgcn_readlane(pos, 63);
+    }
+  }
+  return n;
+}
+
 // tile_slots: dense, the token tiles of M; grouped, the rows of the tile table
 // (max_tiles), which bounds the device-side count a.ntiles[0].
-template <int F, int EPI, int RB, int NW, int KS, int D>
+//
+// TB = 2 (grouped FP8): a unit takes up to two consecutive tiles of one expert,
+// so an expert with 17 .. 32 rows streams its weights once instead of twice.
+// Each weight fragment feeds both tiles' MFMAs; the second tile's activations
+// take as many registers again (112 for K = 7168 on 8 waves, of 256), and its
+// MFMAs are skipped where the group holds one tile.  The two tiles' partial
+// sums go through the two reduction buffers in turn.  256 experts of 7168 x
+// 2 * 2048 with 22 rows each (482 table rows): w13 2110 -> 1176 us (6.2 TB/s
+// of weights), w2 1183 -> 670 us; with no second tiles anywhere the table walk
+// and the shorter pipeline cost 0.8 % (w13) and 2.5 % (w2).
+template <int F, int EPI, int RB, int NW, int KS, int D, int TB = 1>
 __global__ __launch_bounds__(NW * 64) void stream_gemm_kernel(SkinnyArgs a, int tile_slots) {
-  using C = StreamCfg<F, RB, NW, KS, D>;
+  using C = StreamCfg<F, RB, NW, KS, D, TB>;
   constexpr int ROWB = StreamFmt<F>::kRowB;
   constexpr int NI = StreamFmt<F>::kInstr;
   constexpr int L = C::kLoads;
@@ -197,6 +244,11 @@ __global__ __launch_bounds__(NW * 64) void stream_gemm_kernel(SkinnyArgs a, int 
   // GateUp 34.9 -> 34.4 us, LMHead 192.5 -> 189.0 us; the 8-wave split-K
   // products and the FP8 kernels measured no gain).  They need units of an even
   // number of K-steps (step parity = item parity) and >= 3 ring stages.
+  // Read the fragments of step s + 1 while step s computes.  Not for TB = 2:
+  // the second set of fragments spills beside two tiles' activations (w13), or
+  // goes through accumulation registers (w2: 728 against 670 us at 22 rows per
+  // expert).
+  constexpr bool AHEAD = TB == 1;
   constexpr bool PAIR = F == kBF16 && NW == 4 && KS % 2 == 0 && D >= 3;
   static_assert(!C::kInterleave || first_unit_waits_ok<C::kLoads, C::kXLoads, C::kSclLoads, KS, D, PAIR>(),
                 "first unit: a counted wait leaves its item in flight");
@@ -215,7 +267,19 @@ __global__ __launch_bounds__(NW * 64) void stream_gemm_kernel(SkinnyArgs a, int 
   // ---- this work-group's units
   // The grouped count is clamped to the table's rows: the host's launch plan
   // (units per work-group, the LDS span of the table) assumes ntiles <= max_tiles.
-  const int ntiles = grouped ? min(max(__builtin_amdgcn_readfirstlane(a.ntiles[0]), 0), tile_slots) : tile_slots;
+  int ntiles = grouped ? min(max(__builtin_amdgcn_readfirstlane(a.ntiles[0]), 0), tile_slots) : tile_slots;
+  const int table_rows = ntiles;
+  uint16_t* lead = reinterpret_cast<uint16_t*>(lds + C::kLeadOff);
+  if constexpr (TB > 1) {
+    // The units below run over the groups (at most as many as table rows).
+    int* count = reinterpret_cast<int*>(lds + C::kLeadOff + kStreamPairTiles * 2);
+    if (wave == 0) {
+      const int n = group_tiles<TB>(a.tiles, ntiles, lane, lead);
+      if (lane == 0) *count = n;
+    }
+    __syncthreads();
+    ntiles = __builtin_amdgcn_readfirstlane(*count);
+  }
   // bf16 dense split-K: work item u = split * (ntiles * units_n) + unit; the
   // item's waves cover K-steps [(split * NW + kw) * KS, ... + KS).
   const int nsplit = (F == kBF16 && !grouped && a.partial != nullptr) ? a.ksplit : 1;
@@ -244,7 +308,21 @@ __global__ __launch_bounds__(NW * 64) void stream_gemm_kernel(SkinnyArgs a, int 
   const int t_first = (u_begin % units_per_split) / a.units_n;  // grouped: nsplit == 1
   if (grouped) {
     const int t_last = (u_end - 1) / a.units_n;
-    for (int i = threadIdx.x; i < 3 * (t_last - t_first + 1); i += NW * 64) tinfo[i] = a.tiles[3 * t_first + i];
+    if constexpr (TB == 1) {
+      for (int i = threadIdx.x; i < 3 * (t_last - t_first + 1); i += NW * 64) tinfo[i] = a.tiles[3 * t_first + i];
+    } else {
+      for (int i = threadIdx.x; i <= t_last - t_first; i += NW * 64) {
+        const int g0 = lead[t_first + i];
+        const int g1 = t_first + i + 1 < ntiles ? lead[t_first + i + 1] : table_rows;  // one past the group
+        tinfo[C::kTileInts * i] = a.tiles[3 * g0];
+#pragma unroll
+        for (int b = 0; b < TB; ++b) {
+          const int row = min(g0 + b, g1 - 1);
+          tinfo[C::kTileInts * i + 1 + 2 * b] = a.tiles[3 * row + 1];
+          tinfo[C::kTileInts * i + 2 + 2 * b] = g0 + b < g1 ? a.tiles[3 * row + 2] : 0;
+        }
+      }
+    }
     __syncthreads();
   }
 
@@ -253,7 +331,7 @@ __global__ __launch_bounds__(NW * 64) void stream_gemm_kernel(SkinnyArgs a, int 
     if constexpr (EPI == kSilu) return rb == 0 ? nu * 16 : N / 2 + nu * 16;
     else return (nu * RB + rb) * 16;
   };
-  auto tile_expert = [&](int tile) { return grouped ? tinfo[3 * (tile - t_first)] : 0; };
+  auto tile_expert = [&](int tile) { return grouped ? tinfo[C::kTileInts * (tile - t_first)] : 0; };
 
   // ---- DMA issue cursor (uniform): unit iu, K-step is of this wave.
   // Lane offsets inside a 16-row block are the same for every unit.
@@ -340,49 +418,57 @@ __global__ __launch_bounds__(NW * 64) void stream_gemm_kernel(SkinnyArgs a, int 
 
   // ---- activations of the current token tile (registers), per K-step of this wave
   constexpr int XV = (F == kFP8) ? 2 : 4;
-  u32x4 xv[KS][XV];
-  float sx[KS];
+  u32x4 xv[TB][KS][XV];
+  float sx[TB][KS];
   int cur_tile = -1;
-  int my_pair = 0;  // grouped: routed pair of token column r (from sorted_pair)
-  int nrows = 0, row0 = 0;
+  int my_pair[TB] = {};  // grouped: routed pair of token column r (from sorted_pair)
+  int nrows[TB] = {}, row0[TB] = {};
   int cur_split = -1;
-  int tok = 0;  // activation row of this lane's token column
+  int tok[TB] = {};  // activation row of this lane's token column
+  bool two = false;  // TB = 2: the group has a second tile
   auto set_tile = [&](int u) {
     const int split = u / units_per_split;
     const int tile = (u % units_per_split) / a.units_n;
     cur_tile = tile;
     cur_split = split;
-    if (grouped) {
-      row0 = tinfo[3 * (tile - t_first) + 1];
-      nrows = tinfo[3 * (tile - t_first) + 2];
-    } else {
-      row0 = tile * 16;
-      nrows = min(16, a.M - row0);
+#pragma unroll
+    for (int b = 0; b < TB; ++b) {
+      if (grouped) {
+        row0[b] = tinfo[C::kTileInts * (tile - t_first) + 1 + 2 * b];
+        nrows[b] = tinfo[C::kTileInts * (tile - t_first) + 2 + 2 * b];
+      } else {
+        row0[b] = tile * 16;
+        nrows[b] = min(16, a.M - row0[b]);
+      }
+      // columns >= nrows compute garbage, never stored (a zero-row tile reads row row0)
+      const int tcol = max(0, min(r, nrows[b] - 1));
+      tok[b] = row0[b] + tcol;
+      if (grouped) {
+        my_pair[b] = a.sorted_pair[row0[b] + tcol];
+        tok[b] = my_pair[b] / a.topk;
+      }
     }
-    // columns >= nrows compute garbage, never stored (a zero-row tile reads row row0)
-    const int tcol = max(0, min(r, nrows - 1));
-    tok = row0 + tcol;
-    if (grouped) {
-      my_pair = a.sorted_pair[row0 + tcol];
-      tok = my_pair / a.topk;
-    }
+    if constexpr (TB > 1) two = __builtin_amdgcn_readfirstlane(nrows[TB - 1]) > 0;
   };
   // Activations of this wave's K-step k of the current tile and split:
   // C::kXLoads vector loads.
   auto load_x = [&](int k) {
     const int ks = (cur_split * NW + kw) * KS + k;
-    if constexpr (F == kFP8) {
-      const uint8_t* xp = a.x + (size_t)tok * K + (size_t)ks * 128 + 32 * g;
-      xv[k][0] = ld_u32x4(xp);
-      xv[k][1] = ld_u32x4(xp + 16);
-      sx[k] = a.x_scale[(size_t)tok * nkb + ks];
-    } else {
-      const uint8_t* xp = a.x + ((size_t)tok * K + (size_t)ks * 128 + 32 * g) * 2;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) xv[k][j] = ld_u32x4(xp + 16 * j);
+    for (int b = 0; b < TB; ++b) {
+      if constexpr (F == kFP8) {
+        const uint8_t* xp = a.x + (size_t)tok[b] * K + (size_t)ks * 128 + 32 * g;
+        xv[b][k][0] = ld_u32x4(xp);
+        xv[b][k][1] = ld_u32x4(xp + 16);
+        sx[b][k] = a.x_scale[(size_t)tok[b] * nkb + ks];
+      } else {
+        const uint8_t* xp = a.x + ((size_t)tok[b] * K + (size_t)ks * 128 + 32 * g) * 2;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) xv[b][k][j] = ld_u32x4(xp + 16 * j);
+      }
     }
   };
-  f32x4 acc[RB];
+  f32x4 acc[TB][RB];
   int buf = 0;
 
   // One unit.  FIRST: the work-group's first unit with more to follow, its
@@ -397,7 +483,9 @@ __global__ __launch_bounds__(NW * 64) void stream_gemm_kernel(SkinnyArgs a, int 
     const int tile = (u % units_per_split) / a.units_n;
     const int nu = u % a.units_n;
 #pragma unroll
-    for (int rb = 0; rb < RB; ++rb) acc[rb] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int b = 0; b < TB; ++b)
+#pragma unroll
+      for (int rb = 0; rb < RB; ++rb) acc[b][rb] = f32x4{0.f, 0.f, 0.f, 0.f};
     if (!first && (tile != cur_tile || split != cur_split)) {
       set_tile(u);
 #pragma unroll
@@ -428,23 +516,36 @@ __global__ __launch_bounds__(NW * 64) void stream_gemm_kernel(SkinnyArgs a, int 
     };
     auto compute = [&](const StepFrag<F, RB>& fr, auto sc) {
       constexpr int s = decltype(sc)::value;
+      static_for<0, RB>([&](auto rc) {
+        constexpr int rb = decltype(rc)::value;
+        if constexpr (TB > 1 && KS >= 7) {
+          // Each row block widens the activations anew: the widened copies would
+          // take 16 registers more than the wave has.
 #pragma unroll
-      for (int rb = 0; rb < RB; ++rb) {
-        if constexpr (F == kBF16) {
-#pragma unroll
-          for (int j = 0; j < 4; ++j) acc[rb] = mfma_bf16_16x16x32(fr.w[rb][j], xv[s][j], acc[rb]);
-        } else if constexpr (F == kFP8) {
-          const f32x4 part = fp8_block_16x16x128(fr.w[rb][0], fr.w[rb][1], xv[s][0], xv[s][1]);
-          const float scl = sx[s] * fr.sv[rb];
-#pragma unroll
-          for (int i = 0; i < 4; ++i) acc[rb][i] = fmaf(part[i], scl, acc[rb][i]);
-        } else {
-          const Int4Scale ks4 = int4_scale(fr.sv[rb]);
-#pragma unroll
-          for (int j = 0; j < 4; ++j)
-            acc[rb] = mfma_bf16_16x16x32(dequant_int4x8(fr.w[rb][0][j], ks4), xv[s][j], acc[rb]);
+          for (int b = 0; b < TB; ++b) asm volatile("" : "+v"(xv[b][s][0]), "+v"(xv[b][s][1]));
         }
-      }
+        auto tile = [&](auto bc) {
+          constexpr int b = decltype(bc)::value;
+          if constexpr (F == kBF16) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) acc[b][rb] = mfma_bf16_16x16x32(fr.w[rb][j], xv[b][s][j], acc[b][rb]);
+          } else if constexpr (F == kFP8) {
+            const f32x4 part = fp8_block_16x16x128(fr.w[rb][0], fr.w[rb][1], xv[b][s][0], xv[b][s][1]);
+            const float scl = sx[b][s] * fr.sv[rb];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) acc[b][rb][i] = fmaf(part[i], scl, acc[b][rb][i]);
+          } else {
+            const Int4Scale ks4 = int4_scale(fr.sv[rb]);
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+              acc[b][rb] = mfma_bf16_16x16x32(dequant_int4x8(fr.w[rb][0][j], ks4), xv[b][s][j], acc[b][rb]);
+          }
+        };
+        tile(IntC<0>{});
+        if constexpr (TB > 1) {
+          if (two) tile(IntC<1>{});
+        }
+      });
     };
 
     // Software pipeline over the unit's K-steps: the fragments of step s+1 are
@@ -465,7 +566,13 @@ __global__ __launch_bounds__(NW * 64) void stream_gemm_kernel(SkinnyArgs a, int 
       constexpr int s = decltype(sc)::value;
       const int it = (u - u_begin) * KS + s;
       StepFrag<F, RB> nxt;
-      if constexpr (s + 1 < KS) {
+      if constexpr (!AHEAD && s > 0) {
+        constexpr int NY = D - 1;
+        wait_items<L, SI, KS, s, NY>(min(NY, n_items - 1 - it));
+        __builtin_amdgcn_sched_barrier(0);
+        load_frag(cur, it % D, s);
+      }
+      if constexpr (AHEAD && s + 1 < KS) {
         // Wait for step s+1's stage (items issued after it may stay in flight:
         // D - 2, one fewer after an even step when refills go out in pairs).
         constexpr int NY = ring_younger(D, PAIR, s);
@@ -518,55 +625,64 @@ __global__ __launch_bounds__(NW * 64) void stream_gemm_kernel(SkinnyArgs a, int 
         }
       }
       __builtin_amdgcn_sched_barrier(0);
-      if constexpr (s + 1 < KS) cur = nxt;
+      if constexpr (AHEAD && s + 1 < KS) cur = nxt;
     });
 
     // ---- unit end: cross-wave K reduction through LDS, then the epilogue.
     // Each wave's partial goes to the slot of its K-range, so the sums below
     // add the K-ranges in order whatever the rotation.
-    float* rb_base = red + buf * (C::kRed / 4);
+    auto finish = [&](auto bc) {
+      constexpr int b = decltype(bc)::value;
+      float* rb_base = red + buf * (C::kRed / 4);
 #pragma unroll
-    for (int rb = 0; rb < RB; ++rb)
+      for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) rb_base[(kw * RB + rb) * kRedBlock + r * kRedStride + 4 * g + i] = acc[rb][i];
-    wait_lgkm0();
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_sched_barrier(0);
-    if constexpr (EPI == kStore) {
-      for (int idx = threadIdx.x; idx < RB * 256; idx += NW * 64) {
-        const int part = idx >> 8, t = (idx >> 4) & 15, row = idx & 15;
-        float v = 0.f;
+        for (int i = 0; i < 4; ++i) rb_base[(kw * RB + rb) * kRedBlock + r * kRedStride + 4 * g + i] = acc[b][rb][i];
+      wait_lgkm0();
+      __builtin_amdgcn_s_barrier();
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (EPI == kStore) {
+        for (int idx = threadIdx.x; idx < RB * 256; idx += NW * 64) {
+          const int part = idx >> 8, t = (idx >> 4) & 15, row = idx & 15;
+          float v = 0.f;
 #pragma unroll
-        for (int w = 0; w < NW; ++w) v += rb_base[(w * RB + part) * kRedBlock + t * kRedStride + row];
-        // dense: token row; grouped: the routed pair of column t (held by lane t;
-        // every wave runs this loop a uniform number of times)
-        const int orow = grouped ? __shfl(my_pair, t, 64) : row0 + t;
-        const size_t o = (size_t)orow * N + block_row(nu, part) + row;
-        if (t < nrows) {
-          if (nsplit > 1) {
-            a.partial[(size_t)split * a.M * N + o] = v;  // summed (+ residual) by the reduce kernel
-          } else {
-            if (a.residual) v += bf16_bits_to_f32(a.residual[o]);
-            a.out[o] = f32_to_bf16_bits(v);
+          for (int w = 0; w < NW; ++w) v += rb_base[(w * RB + part) * kRedBlock + t * kRedStride + row];
+          // dense: token row; grouped: the routed pair of column t (held by lane t;
+          // every wave runs this loop a uniform number of times)
+          const int orow = grouped ? __shfl(my_pair[b], t, 64) : row0[b] + t;
+          const size_t o = (size_t)orow * N + block_row(nu, part) + row;
+          if (t < nrows[b]) {
+            if (nsplit > 1) {
+              a.partial[(size_t)split * a.M * N + o] = v;  // summed (+ residual) by the reduce kernel
+            } else {
+              if (a.residual) v += bf16_bits_to_f32(a.residual[o]);
+              a.out[o] = f32_to_bf16_bits(v);
+            }
           }
         }
-      }
-    } else {
-      const int idx = threadIdx.x;
-      const int t = (idx >> 4) & 15, row = idx & 15;
-      // pair of token column t: held by lane t of every wave
-      const int pair = __shfl(my_pair, t, 64);
-      if (idx < 256 && t < nrows) {
-        float gs = 0.f, us = 0.f;
+      } else {
+        const int idx = threadIdx.x;
+        const int t = (idx >> 4) & 15, row = idx & 15;
+        // pair of token column t: held by lane t of every wave
+        const int pair = __shfl(my_pair[b], t, 64);
+        if (idx < 256 && t < nrows[b]) {
+          float gs = 0.f, us = 0.f;
 #pragma unroll
-        for (int w = 0; w < NW; ++w) {
-          gs += rb_base[(w * RB + 0) * kRedBlock + t * kRedStride + row];
-          us += rb_base[(w * RB + 1) * kRedBlock + t * kRedStride + row];
+          for (int w = 0; w < NW; ++w) {
+            gs += rb_base[(w * RB + 0) * kRedBlock + t * kRedStride + row];
+            us += rb_base[(w * RB + 1) * kRedBlock + t * kRedStride + row];
+          }
+          a.out[(size_t)pair * (N / 2) + nu * 16 + row] = f32_to_bf16_bits(silu_mul(gs, us));
         }
-        a.out[(size_t)pair * (N / 2) + nu * 16 + row] = f32_to_bf16_bits(silu_mul(gs, us));
       }
+      // The other buffer takes the next sums: every wave has read this one
+      // before it passes the barrier of the sums after those.
+      buf ^= 1;
+    };
+    finish(IntC<0>{});
+    if constexpr (TB > 1) {
+      if (two) finish(IntC<1>{});
     }
-    buf ^= 1;
   };
   // First token tile.  With at least two units, the activations of each K-step
   // go out right before its weight item (the ring prologue and the first
@@ -601,11 +717,11 @@ __global__ __launch_bounds__(NW * 64) void stream_gemm_kernel(SkinnyArgs a, int 
   for (int u = u_next; u < u_end; ++u) run_unit(IntC<0>{}, u);
 }
 
-template <int F, int EPI, int RB, int NW, int KS, int D>
+template <int F, int EPI, int RB, int NW, int KS, int D, int TB = 1>
 static int launch_stream(const SkinnyArgs& a, int tile_slots, int grid, hipStream_t st) {
-  using C = StreamCfg<F, RB, NW, KS, D>;
-  FERRET_HIP_CHECK((set_lds_limit_once<stream_gemm_kernel<F, EPI, RB, NW, KS, D>>(C::kLds)));
-  hipLaunchKernelGGL((stream_gemm_kernel<F, EPI, RB, NW, KS, D>), dim3(grid), dim3(NW * 64), C::kLds, st, a,
+  using C = StreamCfg<F, RB, NW, KS, D, TB>;
+  FERRET_HIP_CHECK((set_lds_limit_once<stream_gemm_kernel<F, EPI, RB, NW, KS, D, TB>>(C::kLds)));
+  hipLaunchKernelGGL((stream_gemm_kernel<F, EPI, RB, NW, KS, D, TB>), dim3(grid), dim3(NW * 64), C::kLds, st, a,
                      tile_slots);
   return (int)hipGetLastError();
 }

@@ -11,7 +11,8 @@
 
 namespace ferret {
 
-constexpr int kStreamMaxTiles = 64;  // token tiles one work-group may touch (tile table in LDS)
+constexpr int kStreamMaxTiles = 64;  // token tiles (or groups of them) one work-group may touch (table in LDS)
+constexpr int kStreamPairTiles = 2048;  // table rows of the kernel that pairs tiles (their group starts in LDS)
 
 struct StreamPlan {
   bool ok = false;      // false: the shape is not covered (the caller uses the per-unit kernel)

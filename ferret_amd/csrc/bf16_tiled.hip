@@ -1,0 +1,213 @@
+// LDS-tiled bf16 product for gfx950, y[M,N] = x[M,K] . w[N,K]^T (+ residual),
+// past the 16 tokens that a unit of the stream kernel holds.
+//
+// HBM-bound on the weights up to about 100 tokens.  A work-group of 8 waves
+// takes RT x 16 weight rows by all tokens (TT x 16) over one K split; both
+// operands go global -> LDS in stages of 128 K (256 bytes of each row, whole
+// lines) through a ring of NS stages, one barrier per stage.  Weights are read
+// once per work-group, the tokens once per row tile (from L2), so RT is the
+// larger of two sizes wherever the row tiles still fill the CUs.  The waves
+// split the K of a stage as well as the tile (WK), which keeps the fragment
+// reads near one LDS read per MFMA at small tiles; the parts meet in LDS once.
+//
+// Every work-group starts at another K-step (row tile index modulo its steps)
+// and wraps around: in lockstep, all of them read the same columns of rows a
+// power of two apart, which sit on few of the memory channels (24576 x 4096 at
+// 64 tokens: 46.6 -> 37.3 us, 34.0 with the weights non-temporal).
+//
+// Measured, start to now (the 16-token stream kernel once per 16 tokens):
+// 4096 x 12288 + residual at 48 tokens 53.4 -> 23 us, 24576 x 4096 at 64 tokens
+// 77.0 -> 34.2 us, at 128 tokens 141.6 -> 51.6 us.
+#include "common.hpp"
+#include "bf16_tiled.hpp"
+
+namespace ferret {
+namespace bt {
+
+// 8 waves: WR along the rows, WT along the tokens, WK along the K of a stage.
+template <int RT, int TT, int KS, int NS, int WR, int WT, int WK>
+struct Cfg {
+  static constexpr int kRows = 16 * RT, kToks = 16 * TT;
+  static constexpr int kRowB = KS * 2;                         // bytes of a stage row
+  static constexpr int kStage = (RT + TT) * 16 * kRowB;
+  static constexpr int kInstr = kStage / 1024;                 // 1-KB loads of a stage: weights, then tokens
+  static constexpr int kWInstr = RT * 16 * kRowB / 1024;
+  static constexpr int kIRows = 1024 / kRowB;                  // rows of a load
+  static constexpr int kLd = (kInstr + 7) / 8;                 // loads per wave (past kInstr: the last one again)
+  static constexpr int kRB = RT / WR, kTB = TT / WT, kKB = KS / 32 / WK;  // row and token blocks, MFMAs deep, per wave
+  static constexpr int kPitch = kRows + 4;                     // floats of a token row of the epilogue
+  static constexpr int kEpi = WK * kToks * kPitch * 4;
+  static constexpr int kLds = NS * kStage > kEpi ? NS * kStage : kEpi;
+  static_assert(WR * WT * WK == 8 && RT % WR == 0 && TT % WT == 0 && (KS / 32) % WK == 0, "8 waves");
+  static_assert(kStage % 1024 == 0 && kLds <= 160 * 1024, "LDS budget");
+  static_assert(NS >= 2 && (NS - 2) * kLd < 63, "vmcnt range");
+};
+
+// Slot of 16-byte chunk c of stage row `row`: the 16 rows of a fragment read
+// fall on distinct banks.
+template <int KS>
+__device__ __forceinline__ int swz(int row, int c) {
+  return KS == 128 ? c ^ (((row & 7) << 1) | ((row >> 3) & 1)) : c ^ ((row & 7) ^ ((row >> 3) & 1));
+}
+
+// Wait until at most min(n, N) stages of L loads are in flight.
+template <int L, int N>
+__device__ __forceinline__ void wait_younger(int n) {
+  if constexpr (N == 0) {
+    wait_vmcnt<0>();
+  } else {
+    if (n >= N) wait_vmcnt<N * L>();
+    else wait_younger<L, N - 1>(n);
+  }
+}
+
+template <int RT, int TT, int KS, int NS, int WR, int WT, int WK>
+__global__ __launch_bounds__(512) void bf16_tiled_kernel(Args p) {
+  using C = Cfg<RT, TT, KS, NS, WR, WT, WK>;
+  extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r = lane & 15, g = lane >> 4;
+  const int wr = wave % WR, wt = (wave / WR) % WT, wk = wave / (WR * WT);
+
+  // Splits vary fastest: with 2, 4 or 8 of them an XCD (work-groups are dealt
+  // to the 8 round-robin) reads one K-range of the tokens only.
+  const int split = blockIdx.x % p.splits;
+  const int tile = blockIdx.x / p.splits;
+  const int tt = tile % p.tok_tiles, rt = tile / p.tok_tiles;
+  const int nkb = p.K / KS;
+  const int k0 = (int)((long long)split * nkb / p.splits), k1 = (int)((long long)(split + 1) * nkb / p.splits);
+  const int nsteps = k1 - k0;
+  const int rot = nsteps > 0 ? (int)((unsigned)(p.rt0 + rt) % (unsigned)nsteps) : 0;
+  const int row0 = rt * C::kRows, tok0 = tt * C::kToks;
+
+  const uint8_t* src[C::kLd];
+  int dst[C::kLd];
+#pragma unroll
+  for (int i = 0; i < C::kLd; ++i) {
+    const int j = min(wave * C::kLd + i, C::kInstr - 1);
+    constexpr int LR = 64 / C::kIRows;         // lanes of a row
+    const int lr = C::kIRows * j + lane / LR;  // stage row
+    const int c = swz<KS>(lr & 15, lane % LR);
+    const bool is_w = j < C::kWInstr;
+    // rows past N or M repeat the last one (never stored)
+    const size_t row = is_w ? min(row0 + lr, p.N - 1) : min(tok0 + lr - C::kRows, p.M - 1);
+    src[i] = (is_w ? p.w : p.x) + (row * p.K + (size_t)k0 * KS) * 2 + c * 16;
+    dst[i] = j * 1024;
+  }
+  auto issue = [&](int step) {
+    uint8_t* st = lds + (step % NS) * C::kStage;
+    const int ks = step + rot < nsteps ? step + rot : step + rot - nsteps;
+#pragma unroll
+    for (int i = 0; i < C::kLd; ++i) {
+      if (p.nt && wave * C::kLd + i < C::kWInstr) g2l_16_nt(src[i] + (size_t)ks * C::kRowB, st + dst[i]);
+      else g2l_16(src[i] + (size_t)ks * C::kRowB, st + dst[i]);
+    }
+  };
+
+  f32x4 acc[C::kRB][C::kTB];
+#pragma unroll
+  for (int a = 0; a < C::kRB; ++a)
+#pragma unroll
+    for (int b = 0; b < C::kTB; ++b) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+#pragma unroll
+  for (int s = 0; s < NS - 1; ++s)
+    if (s < nsteps) issue(s);
+  for (int step = 0; step < nsteps; ++step) {
+    // This stage has landed for every wave, and the slot of the stage before
+    // (the one refilled below) has been read by every wave.
+    wait_younger<C::kLd, NS - 2>(nsteps - 1 - step);
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    if (step + NS - 1 < nsteps) issue(step + NS - 1);
+    __builtin_amdgcn_sched_barrier(0);
+    const uint8_t* st = lds + (step % NS) * C::kStage;
+#pragma unroll
+    for (int k = 0; k < C::kKB; ++k) {
+      const int c = swz<KS>(r, 4 * (wk * C::kKB + k) + g) << 4;
+      u32x4 wf[C::kRB], xf[C::kTB];
+#pragma unroll
+      for (int a = 0; a < C::kRB; ++a)
+        wf[a] = *reinterpret_cast<const u32x4*>(st + ((wr * C::kRB + a) * 16 + r) * C::kRowB + c);
+#pragma unroll
+      for (int b = 0; b < C::kTB; ++b)
+        xf[b] = *reinterpret_cast<const u32x4*>(st + (C::kRows + (wt * C::kTB + b) * 16 + r) * C::kRowB + c);
+#pragma unroll
+      for (int a = 0; a < C::kRB; ++a)
+#pragma unroll
+        for (int b = 0; b < C::kTB; ++b) acc[a][b] = mfma_bf16_16x16x32(wf[a], xf[b], acc[a][b]);
+    }
+  }
+
+  // Epilogue through the idle ring: [K part][token][row], then four outputs of
+  // a token per thread, the parts in order.
+  __builtin_amdgcn_sched_barrier(0);
+  __syncthreads();
+  float* red = reinterpret_cast<float*>(lds);
+#pragma unroll
+  for (int a = 0; a < C::kRB; ++a)
+#pragma unroll
+    for (int b = 0; b < C::kTB; ++b)
+      *reinterpret_cast<f32x4*>(red + (wk * C::kToks + (wt * C::kTB + b) * 16 + r) * C::kPitch +
+                                (wr * C::kRB + a) * 16 + 4 * g) = acc[a][b];
+  __syncthreads();
+  constexpr int Q = C::kRows / 4;
+  for (int i = threadIdx.x; i < C::kToks * Q; i += 512) {
+    const int t = i / Q, q = i % Q, n = row0 + 4 * q;
+    if (tok0 + t >= p.M || n >= p.N) continue;
+    f32x4 v = *reinterpret_cast<const f32x4*>(red + t * C::kPitch + 4 * q);
+#pragma unroll
+    for (int k = 1; k < WK; ++k) v += *reinterpret_cast<const f32x4*>(red + (k * C::kToks + t) * C::kPitch + 4 * q);
+    if (p.splits > 1) {  // summed (+ residual) by the reduce kernel
+      *reinterpret_cast<f32x4*>(p.partial + ((size_t)split * p.M + tok0 + t) * p.N + n) = v;
+    } else {
+      const size_t o = (size_t)(tok0 + t) * p.ldo + n;
+      if (p.residual) {
+        const u32x2 s = *reinterpret_cast<const u32x2*>(p.residual + o);
+        v[0] += __uint_as_float(s[0] << 16);
+        v[1] += __uint_as_float(s[0] & 0xffff0000u);
+        v[2] += __uint_as_float(s[1] << 16);
+        v[3] += __uint_as_float(s[1] & 0xffff0000u);
+      }
+      *reinterpret_cast<u32x2*>(p.out + o) = u32x2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+    }
+  }
+}
+
+// Tile I of kTiles, its waves split by WR, WT, WK.
+template <int I, int WR, int WT, int WK>
+static int launch(const Args& p, hipStream_t st) {
+  constexpr Tile t = kTiles[I];
+  using C = Cfg<t.rt, t.tt, t.ks, t.ns, WR, WT, WK>;
+  constexpr auto kernel = bf16_tiled_kernel<t.rt, t.tt, t.ks, t.ns, WR, WT, WK>;
+  FERRET_HIP_CHECK((set_lds_limit_once<bf16_tiled_kernel<t.rt, t.tt, t.ks, t.ns, WR, WT, WK>>(C::kLds)));
+  const int row_tiles = (p.N + C::kRows - 1) / C::kRows;
+  hipLaunchKernelGGL(kernel, dim3(row_tiles * p.tok_tiles * p.splits), dim3(512), C::kLds, st, p);
+  return (int)hipGetLastError();
+}
+
+}  // namespace bt
+}  // namespace ferret
+
+int ferret_bf16_tiled(int tile, const ferret::bt::Args& p, hipStream_t st) {
+  using namespace ferret::bt;
+  static_assert(kNumTiles == 13, "one case per tile");
+  switch (tile) {
+    case 0: return launch<0, 2, 1, 4>(p, st);
+    case 1: return launch<1, 2, 1, 4>(p, st);
+    case 2: return launch<2, 2, 1, 4>(p, st);
+    case 3: return launch<3, 2, 1, 4>(p, st);
+    case 4: return launch<4, 2, 1, 4>(p, st);
+    case 5: return launch<5, 2, 1, 4>(p, st);
+    case 6: return launch<6, 2, 2, 2>(p, st);
+    case 7: return launch<7, 2, 2, 2>(p, st);
+    case 8: return launch<8, 2, 2, 2>(p, st);
+    case 9: return launch<9, 2, 2, 2>(p, st);
+    case 10: return launch<10, 2, 4, 1>(p, st);
+    case 11: return launch<11, 2, 4, 1>(p, st);
+    case 12: return launch<12, 2, 4, 1>(p, st);
+  }
+  return FERRET_ERR_SHAPE;
+}

@@ -23,6 +23,9 @@
 // the INT4 w13 contract (tasks/kimi-moe-w13-int4-grouped-gemm.yaml:68-95,150-167).
 #include "skinny_kernel.hpp"
 #include "stream_kernel.hpp"
+#include "bf16_tiled.hpp"
+
+int ferret_bf16_tiled(int tile, const ferret::bt::Args& p, hipStream_t st);
 
 namespace ferret {
 
@@ -142,23 +145,60 @@ static int launch_skinny(const SkinnyArgs& a, int ntile_slots, hipStream_t st) {
   return FERRET_ERR_SHAPE;
 }
 
-// y[m, n] = bf16(sum_{s < S} partial[s, m, n] (+ residual[m, n])), splits in
-// order; SN > 0: S == SN, all split loads issued before the first add.
+// y[m, n] = bf16(sum_{s < S} partial[s, m, n] (+ residual[m, n])) for the N
+// outputs of row m = blockIdx.y (row strides: partial N, y and residual ldo),
+// splits in order; SN > 0: S == SN, all split loads issued before the first add.
 template <int SN>
-__global__ __launch_bounds__(256) void linear_splitk_reduce_kernel(const float* __restrict__ partial, int S,
-                                                                   long long mn4, const uint16_t* __restrict__ res,
+__global__ __launch_bounds__(256) void linear_splitk_reduce_kernel(const float* __restrict__ partial, int S, int N,
+                                                                   int ldo, const uint16_t* __restrict__ res,
                                                                    uint16_t* __restrict__ y) {
-  for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < mn4; i += (long long)gridDim.x * 256) {
-    f32x4 v = sum_splits<SN>(reinterpret_cast<const f32x4*>(partial), S, (size_t)mn4, (size_t)i);
-    if (res) {
-      const u32x2 r = reinterpret_cast<const u32x2*>(res)[i];
-      v[0] += __uint_as_float(r[0] << 16);
-      v[1] += __uint_as_float(r[0] & 0xffff0000u);
-      v[2] += __uint_as_float(r[1] << 16);
-      v[3] += __uint_as_float(r[1] & 0xffff0000u);
-    }
-    reinterpret_cast<u32x2*>(y)[i] = u32x2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+  const int n4 = N / 4;
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= n4) return;
+  f32x4 v = sum_splits<SN>(reinterpret_cast<const f32x4*>(partial), S, (size_t)gridDim.y * n4,
+                           (size_t)blockIdx.y * n4 + i);
+  const size_t o = (size_t)blockIdx.y * ldo + (size_t)i * 4;
+  if (res) {
+    const u32x2 r = *reinterpret_cast<const u32x2*>(res + o);
+    v[0] += __uint_as_float(r[0] << 16);
+    v[1] += __uint_as_float(r[0] & 0xffff0000u);
+    v[2] += __uint_as_float(r[1] << 16);
+    v[3] += __uint_as_float(r[1] & 0xffff0000u);
   }
+  *reinterpret_cast<u32x2*>(y + o) = u32x2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+}
+
+static int launch_splitk_reduce(const float* partial, int S, int M, int N, int ldo, const uint16_t* residual,
+                                uint16_t* out, hipStream_t st) {
+  auto* reduce = S == 2 ? linear_splitk_reduce_kernel<2> : S == 3 ? linear_splitk_reduce_kernel<3>
+               : S == 4 ? linear_splitk_reduce_kernel<4> : linear_splitk_reduce_kernel<0>;
+  hipLaunchKernelGGL(reduce, dim3((N / 4 + 255) / 256, M), dim3(256), 0, st, partial, S, N, ldo, residual, out);
+  return (int)hipGetLastError();
+}
+
+// The LDS-tiled product over weight rows [n0, n0 + n) by `plan`, partials in ws.
+static int launch_bf16_tiled(const bt::Plan& plan, const SkinnyArgs& a, int n0, int n, void* ws, hipStream_t st) {
+  const bt::Tile& t = bt::kTiles[plan.tile];
+  bt::Args p{};
+  p.w = a.w + (size_t)n0 * a.K * 2;
+  p.x = a.x;
+  p.residual = a.residual ? a.residual + n0 : nullptr;
+  p.out = a.out + n0;
+  p.partial = static_cast<float*>(ws);
+  p.M = a.M;
+  p.N = n;
+  p.K = a.K;
+  p.ldo = a.N;
+  p.splits = plan.splits;
+  p.tok_tiles = plan.tok_tiles;
+  p.rt0 = n0 / (16 * t.rt);
+  // Weights that only one work-group reads: past the caches (24576 x 4096 at 64
+  // tokens 37.3 -> 34.0 us, 4096 x 12288 at 32 22.0 -> 20.3); beside the tokens
+  // of a wide split it was slower (4096 x 4096 at 64 tokens 12.0 -> 12.8).
+  p.nt = plan.tok_tiles == 1 && (plan.splits == 1 || t.tt <= 2);
+  const int rc = ferret_bf16_tiled(plan.tile, p, st);
+  if (rc != 0 || plan.splits == 1) return rc;
+  return launch_splitk_reduce(p.partial, p.splits, p.M, p.N, p.ldo, p.residual, p.out, st);
 }
 
 // K splits of the bf16 stream kernel for y = x.W^T: 1 when a work-group per CU
@@ -188,12 +228,37 @@ static int linear_splits(int M, int N, int K) {
   return best;
 }
 
+// The LDS-tiled kernel's plan for the shapes it takes, else none.
+//   * Past 16 tokens: it streams the weights once for all of them, the stream
+//     and per-unit kernels once per 16 (4096 x 12288 at 17 tokens 20.5 against
+//     36.2 us, 24576 x 4096 at 32 32.7 against 45.5, 6144 x 4096 at 32 14.1
+//     against 14.7).
+//   * Up to 16 tokens where the stream kernel does not take K (K / 128 not 2, 4,
+//     7 or 8 per wave; 1536 x 9984: 11.2 against the per-unit kernel's 17.4 us
+//     at one token, 12.1 against 23.4 at 16; 16000 x 1280 9.0 against 10.9 and
+//     9.2 against 14.7).
+//   * Not where the whole product is a few microseconds: a split's second launch
+//     and the ring's fill cost 2-3 us more than the other kernels spend.  In
+//     16-token tiles x N x K the line lies at 2^25 against the stream kernel (4
+//     tiles of 2048 x 2048, 2^24: 9.7 against 7.0 us; 2 of 4096 x 4096, 2^25:
+//     10.4 against 13.9) and at 10 * 2^20 against the per-unit one (2 tiles of
+//     4096 x 640: 5.8 against 5.3; 4: 6.7 against 7.7).
+static bt::Plan tiled_plan(int M, int N, int K) {
+  const int ncu = cu_count();
+  const bool stream = stream_plan(false, 1, 8, N, K, 1, false, linear_splits(M, N, K), ncu).ok ||
+                      (N / 16 >= 4 * ncu && stream_plan(false, 1, 4, N, K, 1, false, 1, ncu).ok);
+  const long long work = (long long)((M + 15) / 16) * N * K;
+  if ((stream && M <= 16) || work < (stream ? 32LL : 10LL) << 20) return bt::Plan{};
+  return bt::plan(M, N, K, ncu);
+}
+
 }  // namespace ferret
 
 using namespace ferret;
 
 size_t ferret_linear_bf16_workspace(int M, int N, int K) {
-  const int s = linear_splits(M, N, K);
+  const bt::Plan tiled = tiled_plan(M, N, K);
+  const int s = tiled.ok ? tiled.splits : linear_splits(M, N, K);
   return s > 1 ? (size_t)s * M * N * sizeof(float) : 0;
 }
 
@@ -212,20 +277,17 @@ extern "C" int ferret_linear_bf16(const void* x, const void* w, const void* resi
   a.N = N;
   a.K = K;
   a.units_n = N / 16;
-  const int splits = linear_splits(M, N, K);
   const size_t need = ferret_linear_bf16_workspace(M, N, K);
+  const bt::Plan tiled = tiled_plan(M, N, K);
+  if (tiled.ok && (need == 0 || (ws != nullptr && ws_bytes >= need))) return launch_bf16_tiled(tiled, a, 0, N, ws, st);
+  const int splits = tiled.ok ? 1 : linear_splits(M, N, K);
   if (splits > 1 && ws != nullptr && ws_bytes >= need && (M * (long long)N) % 4 == 0) {
     a.partial = static_cast<float*>(ws);
     a.ksplit = splits;
     const int rc = try_stream<kBF16, kStore, 1, 3, 8>(a, (M + 15) / 16, 0, st);
     if (rc != 1) {
       if (rc != 0) return rc;
-      const long long mn4 = (long long)M * N / 4;
-      const int grid = (int)std::min<long long>((mn4 + 255) / 256, 4096);
-      auto* reduce = splits == 2 ? linear_splitk_reduce_kernel<2> : splits == 3 ? linear_splitk_reduce_kernel<3>
-                   : splits == 4 ? linear_splitk_reduce_kernel<4> : linear_splitk_reduce_kernel<0>;
-      hipLaunchKernelGGL(reduce, dim3(grid), dim3(256), 0, st, a.partial, splits, mn4, a.residual, a.out);
-      return (int)hipGetLastError();
+      return launch_splitk_reduce(a.partial, splits, M, N, N, a.residual, a.out, st);
     }
     a.partial = nullptr;
     a.ksplit = 0;
@@ -287,11 +349,30 @@ extern "C" int ferret_linear_bf16_noalloc(const void* x, const void* w, const vo
   FERRET_REQUIRE(x && w && y, FERRET_ERR_NULL);
   FERRET_REQUIRE(M >= 1 && N >= 16 && K >= 128, FERRET_ERR_SHAPE);
   FERRET_REQUIRE(N % 16 == 0 && K % 128 == 0 && K / 128 <= 128, FERRET_ERR_SHAPE);
+  const int splits = linear_splits(M, N, K);
+  FERRET_REQUIRE(splits <= 1 || (size_t)splits * M * N * sizeof(float) <= kNoAllocScratchBytes, FERRET_ERR_WORKSPACE);
   const size_t need = ferret_linear_bf16_workspace(M, N, K);
-  FERRET_REQUIRE(need <= kNoAllocScratchBytes, FERRET_ERR_WORKSPACE);
   void* ws = nullptr;
   if (need > 0) FERRET_HIP_CHECK(scratch_address(&ws));
-  return ferret_linear_bf16(x, w, residual, y, M, N, K, ws, need, stream);
+  const bt::Plan tiled = tiled_plan(M, N, K);
+  if (!tiled.ok || need <= kNoAllocScratchBytes) return ferret_linear_bf16(x, w, residual, y, M, N, K, ws, need, stream);
+  // Partials larger than the array: the same plan over runs of whole row tiles
+  // whose partials fit (each output's sums are those of one launch).
+  SkinnyArgs a{};
+  a.w = static_cast<const uint8_t*>(w);
+  a.x = static_cast<const uint8_t*>(x);
+  a.residual = static_cast<const uint16_t*>(residual);
+  a.out = static_cast<uint16_t*>(y);
+  a.M = M;
+  a.N = N;
+  a.K = K;
+  const int tile_rows = 16 * bt::kTiles[tiled.tile].rt;
+  const int rows = (int)(kNoAllocScratchBytes / ((size_t)tiled.splits * M * sizeof(float))) / tile_rows * tile_rows;
+  for (int n0 = 0; n0 < N; n0 += rows) {
+    const int rc = launch_bf16_tiled(tiled, a, n0, std::min(rows, N - n0), ws, (hipStream_t)stream);
+    if (rc != 0) return rc;
+  }
+  return FERRET_OK;
 }
 
 extern "C" void launch_gemv(void* input, void* weight, void* residual, void* output, int N, int K,

@@ -57,9 +57,9 @@ void launch_gemv(void* input, void* weight, void* residual, void* output, int N,
  * Requirements: 1 <= M, N % 16 == 0, K % 128 == 0, K/128 <= 128.
  * `ws` (optional): with at least ferret_workspace_bytes(0, M, N, K, 0) bytes
  * (non-zero when splitting K evens out the work over the CUs, e.g. N = 6144 or
- * K = 12288 at M <= 16) the product runs split-K: fp32 partials in the
- * workspace, summed in split order (+ residual) by a second kernel
- * (deterministic); with NULL the same result comes unsplit.
+ * K = 12288) the product runs split-K: fp32 partials in the workspace, summed
+ * in split order (+ residual) by a second kernel (deterministic); with NULL the
+ * same result comes unsplit (past 16 tokens more slowly).
  */
 int ferret_linear_bf16(const void* x, const void* w, const void* residual, void* y, int M, int N,
                        int K, void* ws, size_t ws_bytes, void* stream);
@@ -70,9 +70,11 @@ int ferret_linear_bf16(const void* x, const void* w, const void* residual, void*
  * under HIP graph capture, tight serving loops, harnesses that forbid
  * hipMalloc).  Shapes that run split-K take their fp32 partials from a
  * library-owned device array of ferret_linear_bf16_noalloc_max_bytes()
- * (4 MiB) per GPU; a shape needing more (ferret_workspace_bytes(0, M, N, K, 0)
- * larger than that) is rejected with FERRET_ERR_WORKSPACE.  The result is
- * bit-identical to ferret_linear_bf16 with a workspace.  Calls that overlap on
+ * (4 MiB) per GPU; a shape whose partials by 16-token tiles need more (M = 100,
+ * N = 4096, K = 12288) is rejected with FERRET_ERR_WORKSPACE, and one that
+ * needs more only because it takes all tokens at once (M > 16) runs in several
+ * ranges of weight rows.  The result is bit-identical to ferret_linear_bf16
+ * with a workspace.  Calls that overlap on
  * one GPU (different streams or threads) share the array and race: serialise
  * them.  The array's address is looked up once per device, by the first call
  * of ferret_linear_bf16_noalloc_max_bytes or of this entry point on it: make

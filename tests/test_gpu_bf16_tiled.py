@@ -1,0 +1,65 @@
+"""The LDS-tiled bf16 product: edges of its tiles, its K splits and its entry points.
+
+Against the oracle, at token and row counts on both sides of every tile size,
+K that no power of two divides, and K shorter than the splits; then the
+allocation-free entry against the workspace one, bit for bit, also where the
+partials exceed its array and the product runs in several row ranges.
+"""
+from __future__ import annotations
+
+import pytest
+import torch
+
+from oracle import gemm as G
+from oracle import metrics as MT
+from tests.gpu_helpers import assert_gemm_close, bf16_out, bits16
+
+pytestmark = pytest.mark.gpu
+
+
+def _inputs(M, N, K, res):
+    g = torch.Generator(device="cuda").manual_seed(M * 1000 + N + K)
+    x = torch.randn((M, K), generator=g, device="cuda").to(torch.bfloat16)
+    w = (torch.randn((N, K), generator=g, device="cuda") * 0.05).to(torch.bfloat16)
+    return x, w, torch.randn((M, N), generator=g, device="cuda").to(torch.bfloat16) if res else None
+
+
+# M: one past a tile, exact, one short, several token tiles.  N: remainders of 16, 48, 64 and 80 in the row tiles.
+# K / 128: 1 (fewer steps than stages), 2, 5, 19, 78; up to 16 tokens the shapes the stream kernel leaves.
+@pytest.mark.parametrize("M,N,K,res", [
+    (17, 49168, 128, True), (32, 12304, 640, False), (33, 2128, 2432, True), (48, 5072, 4096, True),
+    (49, 24592, 128, False), (64, 6160, 640, True), (65, 304, 9984, False), (96, 1040, 2432, True),
+    (97, 1552, 4096, False), (128, 2064, 640, True), (129, 528, 2432, False), (255, 688, 1280, True),
+    (300, 1552, 384, False), (1, 1536, 9984, True), (16, 4400, 2432, False), (7, 25008, 640, True),
+    (20, 73744, 256, False), (100, 24592, 256, True), (1000, 48, 2432, False)])
+def test_matches_the_oracle(ops, M, N, K, res):
+    print(f"[case] bf16 tiled M={M} N={N} K={K} res={res}", flush=True)
+    x, w, r = _inputs(M, N, K, res)
+    y = ops.linear_bf16(x, w, r, out=torch.full((M, N), float("nan"), dtype=torch.bfloat16, device="cuda"))
+    torch.cuda.synchronize()
+    ref = G.linear_bf16(bits16(x), bits16(w), bits16(r) if res else None)
+    assert_gemm_close(bf16_out(y), ref, "bf16 tiled")
+    e, nbad = MT.linear_rel_err(bf16_out(y), ref)
+    assert nbad == 0 and e < 5e-3
+
+
+@pytest.mark.parametrize("M,N,K,res", [(20, 4096, 4096, True), (64, 6144, 4096, True), (100, 6144, 4096, False)])
+def test_allocation_free_entry_gives_the_same_bits(hip, M, N, K, res):
+    need = int(hip.ferret_workspace_bytes(0, M, N, K, 0))
+    print(f"[case] bf16 tiled noalloc M={M} N={N} K={K} partials {need}", flush=True)
+    assert need > 0 and hip.ferret_linear_bf16_noalloc_max_bytes() == 4 << 20
+    assert M < 64 or need > 4 << 20          # the last two run in row ranges
+    x, w, r = _inputs(M, N, K, res)
+    ws = torch.empty(need, dtype=torch.uint8, device="cuda")
+    ya, yb = (torch.full((M, N), float("nan"), dtype=torch.bfloat16, device="cuda") for _ in range(2))
+    rp, st = r.data_ptr() if res else None, torch.cuda.current_stream().cuda_stream
+    assert hip.ferret_linear_bf16(x.data_ptr(), w.data_ptr(), rp, ya.data_ptr(), M, N, K, ws.data_ptr(), need, st) == 0
+    assert hip.ferret_linear_bf16_noalloc(x.data_ptr(), w.data_ptr(), rp, yb.data_ptr(), M, N, K, st) == 0
+    torch.cuda.synchronize()
+    assert torch.equal(ya.view(torch.int16), yb.view(torch.int16))
+
+
+@pytest.fixture(scope="module")
+def ops(hip):
+    from ferret_amd import ops as O
+    return O

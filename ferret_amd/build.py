@@ -3,7 +3,9 @@
     python -m ferret_amd.build            # compile every source, link the library
     python -m ferret_amd.build --verbose  # also print kernel register/LDS usage
 
-Objects go to ferret_amd/_build/, the library to ferret_amd/libferret_hip.so.
+Objects go to ferret_amd/_build/, the library to ferret_amd/libferret_hip.so,
+and the native call path of ferret_amd.ops (csrc/native.cpp, a CPython module
+over torch's headers, linked to the library) to ferret_amd/_native.so.
 """
 from __future__ import annotations
 
@@ -19,6 +21,7 @@ ROOT = os.path.dirname(PKG)
 CSRC = os.path.join(PKG, "csrc")
 BUILD = os.path.join(PKG, "_build")
 LIB = os.path.join(PKG, "libferret_hip.so")
+NATIVE = os.path.join(PKG, "_native.so")
 SOURCES = ["skinny.hip", "bf16_tiled.hip", "fp8_tiled.hip", "fp8_square.hip", "routing.hip", "moe_tail.hip", "ue8m0.hip",
            "dispatch.hip"]
 ARCH = "gfx950"
@@ -111,7 +114,30 @@ def build(verbose: bool = False) -> str:
     if res.returncode != 0:
         raise RuntimeError(f"link failed:\n{res.stdout}{res.stderr}")
     os.replace(tmp, LIB)
+    build_native()
     return LIB
+
+
+def build_native() -> str:
+    """Compile csrc/native.cpp (host code only) against torch and the library."""
+    import sysconfig
+
+    import torch
+
+    troot = os.path.dirname(torch.__file__)
+    tmp = NATIVE + ".tmp"
+    cmd = [shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall",
+           "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", f"-I{troot}/include", f"-I{troot}/include/torch/csrc/api/include",
+           f"-I{os.path.join(os.path.dirname(os.path.dirname(hipcc())), 'include')}", "-I/opt/rocm/include",
+           f"-I{sysconfig.get_paths()['include']}",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           os.path.join(CSRC, "native.cpp"), "-o", tmp, f"-L{troot}/lib", "-lc10", "-lc10_hip", "-ltorch_cpu",
+           "-ltorch_python", f"-L{PKG}", "-l:libferret_hip.so", "-Wl,-rpath,$ORIGIN"]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"g++ failed for native.cpp:\n{res.stdout}{res.stderr}")
+    os.replace(tmp, NATIVE)
+    return NATIVE
 
 
 def main() -> int:

@@ -256,10 +256,13 @@ static bt::Plan tiled_plan(int M, int N, int K) {
 
 using namespace ferret;
 
-size_t ferret_linear_bf16_workspace(int M, int N, int K) {
-  const bt::Plan tiled = tiled_plan(M, N, K);
+static size_t linear_workspace(const bt::Plan& tiled, int M, int N, int K) {
   const int s = tiled.ok ? tiled.splits : linear_splits(M, N, K);
   return s > 1 ? (size_t)s * M * N * sizeof(float) : 0;
+}
+
+size_t ferret_linear_bf16_workspace(int M, int N, int K) {
+  return linear_workspace(tiled_plan(M, N, K), M, N, K);
 }
 
 extern "C" int ferret_linear_bf16(const void* x, const void* w, const void* residual, void* y, int M,
@@ -277,8 +280,8 @@ extern "C" int ferret_linear_bf16(const void* x, const void* w, const void* resi
   a.N = N;
   a.K = K;
   a.units_n = N / 16;
-  const size_t need = ferret_linear_bf16_workspace(M, N, K);
   const bt::Plan tiled = tiled_plan(M, N, K);
+  const size_t need = linear_workspace(tiled, M, N, K);
   if (tiled.ok && (need == 0 || (ws != nullptr && ws_bytes >= need))) return launch_bf16_tiled(tiled, a, 0, N, ws, st);
   const int splits = tiled.ok ? 1 : linear_splits(M, N, K);
   if (splits > 1 && ws != nullptr && ws_bytes >= need && (M * (long long)N) % 4 == 0) {
@@ -351,10 +354,10 @@ extern "C" int ferret_linear_bf16_noalloc(const void* x, const void* w, const vo
   FERRET_REQUIRE(N % 16 == 0 && K % 128 == 0 && K / 128 <= 128, FERRET_ERR_SHAPE);
   const int splits = linear_splits(M, N, K);
   FERRET_REQUIRE(splits <= 1 || (size_t)splits * M * N * sizeof(float) <= kNoAllocScratchBytes, FERRET_ERR_WORKSPACE);
-  const size_t need = ferret_linear_bf16_workspace(M, N, K);
+  const bt::Plan tiled = tiled_plan(M, N, K);
+  const size_t need = linear_workspace(tiled, M, N, K);
   void* ws = nullptr;
   if (need > 0) FERRET_HIP_CHECK(scratch_address(&ws));
-  const bt::Plan tiled = tiled_plan(M, N, K);
   if (!tiled.ok || need <= kNoAllocScratchBytes) return ferret_linear_bf16(x, w, residual, y, M, N, K, ws, need, stream);
   // Partials larger than the array: the same plan over runs of whole row tiles
   // whose partials fit (each output's sums are those of one launch).

@@ -64,6 +64,30 @@ class FerretError(RuntimeError):
 
 
 _LIB = None
+_NATIVE = None
+NATIVE_PATH = os.path.join(os.path.dirname(LIB_PATH), "_native.so")
+
+
+class _Absent:
+    """In place of the native call path where neither it nor the library is
+    built: every operator takes its Python path, which says what is missing."""
+
+    def __getattr__(self, name):
+        return lambda *args: None
+
+
+def native():
+    """The native call path of ferret_amd.ops (csrc/native.cpp), loaded once."""
+    global _NATIVE
+    if _NATIVE is None:
+        if not os.path.exists(LIB_PATH):
+            return _Absent()
+        if not os.path.exists(NATIVE_PATH):
+            raise RuntimeError(f"{NATIVE_PATH} is missing: build it with `python -m ferret_amd.build`")
+        load()
+        from . import _native
+        _NATIVE = _native
+    return _NATIVE
 
 
 def load():

@@ -3,6 +3,11 @@
 Every wrapper validates dtype / device / contiguity / shape on the host, passes
 raw device pointers plus the current HIP stream, and raises FerretError on a
 non-zero return code.  There is no CPU path.
+
+The plain case of each operator (contiguous GPU tensors of the right types and
+shapes) runs in native code, checks and allocations included (csrc/native.cpp);
+it answers None for everything else, and the Python code below then names the
+error.
 """
 from __future__ import annotations
 
@@ -13,6 +18,11 @@ import torch
 from . import lib as _lib
 
 FP8 = torch.float8_e4m3fn
+
+
+def _flags_or_none(mma) -> int:
+    """The flag bits of `mma`, -1 (not taken by the native path) where it is invalid."""
+    return 0 if mma == "bf16" else _lib.FP8_MMA_E4M3 if mma == "e4m3" else -1
 
 
 def _stream() -> int:
@@ -64,6 +74,9 @@ def linear_bf16(x: torch.Tensor, w: torch.Tensor, residual: torch.Tensor | None 
     `workspace`, or from torch's caching allocator when none (or a too small
     one) is passed.
     """
+    y = _lib.native().linear_bf16(x, w, residual, out, workspace)
+    if y is not None:
+        return y
     _dev(x, "x", torch.bfloat16, 2)
     _dev(w, "w", torch.bfloat16, 2)
     M, K = x.shape
@@ -110,6 +123,9 @@ def fp8_gemm_blockscale(a: torch.Tensor, sa: torch.Tensor, b: torch.Tensor, sb: 
     taken from torch's caching allocator).  mma="e4m3" opts the tiled (M > 16)
     kernels into the FP8 MFMA (FERRET_FP8_MMA_E4M3: faster, less precise).
     """
+    y = _lib.native().fp8_gemm_blockscale(a, sa, b, sb, out, workspace, _flags_or_none(mma))
+    if y is not None:
+        return y
     _dev(a, "a", (FP8, torch.uint8), 2)
     _dev(b, "b", (FP8, torch.uint8), 2)
     M, K = a.shape
@@ -187,6 +203,9 @@ def fp8_gemm_ue8m0(a: torch.Tensor, sfa: torch.Tensor, b: torch.Tensor, sfb: tor
     expand_block_scales); nk = K/128.  A workspace of fp8_ue8m0_workspace_bytes
     is taken from torch's caching allocator unless one is passed.
     """
+    y = _lib.native().fp8_gemm_ue8m0(a, sfa, b, sfb, out, workspace)
+    if y is not None:
+        return y
     _dev(a, "a", (FP8, torch.uint8), 2)
     _dev(b, "b", (FP8, torch.uint8), 2)
     M, K = a.shape
@@ -216,6 +235,9 @@ def fp8_gemm_ue8m0(a: torch.Tensor, sfa: torch.Tensor, b: torch.Tensor, sfb: tor
 
 def moe_route_topk(logits: torch.Tensor, topk: int, with_weights: bool = True):
     """ids int32 [T, topk] (logit desc, expert asc) and softmax weights [T, topk]."""
+    r = _lib.native().moe_route_topk(logits, topk, with_weights)
+    if r is not None:
+        return r
     T, E = logits.shape
     ids = torch.empty((T, topk), dtype=torch.int32, device=logits.device)
     w = torch.empty((T, topk), dtype=torch.float32, device=logits.device) if with_weights else None
@@ -252,6 +274,10 @@ def moe_permute(ids: torch.Tensor, num_experts: int, tile_m: int | None = None,
     ferret_workspace_bytes(4, P, 0, 0, E) bytes (taken from torch's caching
     allocator unless one at least that large is passed).
     """
+    r = _lib.native().moe_permute(ids, num_experts, tile_m, workspace)
+    if r is not None:
+        counts, offsets, sorted_pair, tiles, ntiles, tile_m, max_tiles, topk, T = r
+        return Routing(counts, offsets, sorted_pair, tiles, ntiles, tile_m, max_tiles, num_experts, topk, T)
     T, topk = ids.shape
     P = T * topk
     if tile_m is None:
@@ -280,6 +306,11 @@ def moe_permute(ids: torch.Tensor, num_experts: int, tile_m: int | None = None,
 def moe_w13_fp8(x: torch.Tensor, sx: torch.Tensor, w: torch.Tensor, sw: torch.Tensor, routing: Routing,
                 out: torch.Tensor | None = None, mma: str = "bf16") -> torch.Tensor:
     """out[P, N/2] bf16 = silu(gate) * up of the FP8 block-scaled w13 projection."""
+    y = _lib.native().moe_w13_fp8(x, sx, w, sw, routing.sorted_pair, routing.tiles, routing.ntiles, routing.max_tiles,
+                                  routing.tile_m, routing.topk, routing.num_experts, routing.num_tokens,
+                                  out, _flags_or_none(mma))
+    if y is not None:
+        return y
     T, K = x.shape
     E, N, K2 = w.shape
     if K2 != K or E != routing.num_experts or T != routing.num_tokens:
@@ -327,6 +358,10 @@ def moe_w13_w4a16(x: torch.Tensor, wq: torch.Tensor, ws: torch.Tensor, routing: 
     wq: the checkpoint words int32 [E, N, K/8], or their tiles from
     int4_tile_weights (int32 [E, N/16, K/128, 16, 16]); the result is the same
     bit for bit."""
+    y = _lib.native().moe_w13_w4a16(x, wq, ws, routing.sorted_pair, routing.tiles, routing.ntiles, routing.max_tiles,
+                                    routing.tile_m, routing.topk, routing.num_experts, routing.num_tokens, out)
+    if y is not None:
+        return y
     T, K = x.shape
     tiled = wq.dim() == 5
     if tiled:
@@ -359,6 +394,9 @@ def moe_w13_w4a16(x: torch.Tensor, wq: torch.Tensor, ws: torch.Tensor, routing: 
 
 def quant_act_e4m3(x: torch.Tensor, q: torch.Tensor | None = None, scale: torch.Tensor | None = None):
     """bf16 x [M, K] -> (e4m3 q [M, K], fp32 scale [M, K/128]) by the 1x128 absmax/448 rule."""
+    r = _lib.native().quant_act_e4m3(x, q, scale)
+    if r is not None:
+        return r
     _dev(x, "x", torch.bfloat16, 2)
     M, K = x.shape
     _same_device(x, q, scale)
@@ -377,6 +415,11 @@ def quant_act_e4m3(x: torch.Tensor, q: torch.Tensor | None = None, scale: torch.
 def moe_w2_fp8(h: torch.Tensor, sh: torch.Tensor, w: torch.Tensor, sw: torch.Tensor, routing: Routing,
                out: torch.Tensor | None = None, mma: str = "bf16") -> torch.Tensor:
     """out[P, N] bf16 (pair order) = the FP8 block-scaled down projection of h [P, K] (pair order)."""
+    y = _lib.native().moe_w2_fp8(h, sh, w, sw, routing.sorted_pair, routing.tiles, routing.ntiles, routing.max_tiles,
+                                 routing.tile_m, routing.topk, routing.num_experts, routing.num_tokens,
+                                 out, _flags_or_none(mma))
+    if y is not None:
+        return y
     P, K = h.shape
     E, N, K2 = w.shape
     if K2 != K or E != routing.num_experts or P != routing.num_tokens * routing.topk:
@@ -398,6 +441,9 @@ def moe_w2_fp8(h: torch.Tensor, sh: torch.Tensor, w: torch.Tensor, sw: torch.Ten
 
 def moe_combine(o: torch.Tensor, weights: torch.Tensor, out: torch.Tensor | None = None) -> torch.Tensor:
     """y[T, N] bf16 = sum_j weights[t, j] * o[t*topk + j] (fp32, j order)."""
+    y = _lib.native().moe_combine(o, weights, out)
+    if y is not None:
+        return y
     T, topk = weights.shape
     P, N = o.shape
     if P != T * topk:

@@ -1,7 +1,7 @@
 // Skinny (<= 16 token) weight-streaming GEMMs for gfx950: bf16 decode linear,
 // small-M FP8 block-scaled GEMM, and the decode-sized MoE grouped GEMMs (FP8
 // w13 and w2, INT4 W4A16 w13) with the fused SiLU(gate)*up epilogue.  Shapes
-// whose K-steps split evenly into 2, 4, 7 or 8 per wave run the persistent
+// whose K-steps split evenly into 2, 4, 7 or 8 per wave (w2 also 3) run the persistent
 // LDS-staged stream kernel of stream_kernel.hpp (bf16 with K split over a
 // workspace where the row units alone would leave CUs idle); the per-unit
 // kernel below takes the rest.
@@ -46,8 +46,9 @@ static int cu_count() {
 // Stream-kernel launch (persistent grid, one work-group of NW waves per CU):
 // returns 1 if the shape is not covered (the caller then uses the per-unit
 // kernel), else the launch status.  KS = K-steps per wave = K / 128 / NW.
-template <int F, int EPI, int RB, int D, int NW = 8>
-static int try_stream(const SkinnyArgs& a_in, int dense_tiles, int max_tiles, hipStream_t st) {
+// `per_cu` work-groups share a CU (fewer waves each).
+template <int F, int EPI, int RB, int D, int NW>
+static int plan_and_launch(const SkinnyArgs& a_in, int dense_tiles, int max_tiles, hipStream_t st, int per_cu) {
   // The unit count, K-steps per wave and tile-table span come from the
   // host-only plan (stream_plan.hpp), which the CPU tests check over every
   // configuration instantiated here: a unit is RB 16-row blocks (SiLU: one
@@ -57,7 +58,7 @@ static int try_stream(const SkinnyArgs& a_in, int dense_tiles, int max_tiles, hi
   const bool grouped = a_in.tiles != nullptr;
   // bf16 dense split-K: each work item covers K / nsplit (see stream_gemm_kernel)
   const int nsplit = (F == kBF16 && !grouped && a_in.partial != nullptr) ? a_in.ksplit : 1;
-  const int grid = cu_count();
+  const int grid = cu_count() * per_cu;
   const StreamPlan plan = stream_plan(EPI == kSilu, RB, NW, a_in.N, a_in.K, grouped ? max_tiles : dense_tiles,
                                       grouped, nsplit, grid);
   if (!plan.ok) return 1;
@@ -74,21 +75,36 @@ static int try_stream(const SkinnyArgs& a_in, int dense_tiles, int max_tiles, hi
     if (a.pair_tiles && max_tiles <= kStreamPairTiles) {
       switch (plan.ks) {
         case 2: return launch_stream<F, EPI, RB, NW, 2, D, 2>(a, slots, grid, st);
-        case 4: return launch_stream<F, EPI, RB, NW, 4, D, 2>(a, slots, grid, st);
+        case 3: if constexpr (RB == 4) return launch_stream<F, EPI, RB, NW, 3, D, 2>(a, slots, grid, st); else break;
+        case 4: if constexpr (NW != 2) return launch_stream<F, EPI, RB, NW, 4, D, 2>(a, slots, grid, st); else break;
         case 7: return launch_stream<F, EPI, RB, NW, 7, D, 2>(a, slots, grid, st);
       }
     }
   }
   switch (plan.ks) {
     case 2: return launch_stream<F, EPI, RB, NW, 2, D2>(a, slots, grid, st);
-    case 4: return launch_stream<F, EPI, RB, NW, 4, D4>(a, slots, grid, st);
+    case 3: if constexpr (RB == 4) return launch_stream<F, EPI, RB, NW, 3, D>(a, slots, grid, st); else return 1;
+    case 4: if constexpr (NW != 2) return launch_stream<F, EPI, RB, NW, 4, D4>(a, slots, grid, st); else return 1;
     // More than 8 waves leave a wave 128 VGPRs (two work-groups' worth of waves
     // on some SIMDs), too few for 7 or 8 K-steps of activations: those shapes
     // take the 8-wave configuration (the caller's fallback).
     case 7: if constexpr (NW <= 8) return launch_stream<F, EPI, RB, NW, 7, D>(a, slots, grid, st); else return 1;
-    case 8: if constexpr (NW <= 8) return launch_stream<F, EPI, RB, NW, 8, D>(a, slots, grid, st); else return 1;
+    case 8: if constexpr (NW <= 8 && NW != 2) return launch_stream<F, EPI, RB, NW, 8, D>(a, slots, grid, st); else return 1;
   }
   return 1;
+}
+
+template <int F, int EPI, int RB, int D, int NW = 8>
+static int try_stream(const SkinnyArgs& a, int dense_tiles, int max_tiles, hipStream_t st) {
+  return plan_and_launch<F, EPI, RB, D, NW>(a, dense_tiles, max_tiles, st, 1);
+}
+
+// Grouped: two work-groups of 2 waves per CU, each in at most half of its LDS,
+// for the K / 128 that 4 waves leave (4, 6 and 14: 2, 3 and 7 K-steps per wave).
+template <int F, int EPI, int RB, int D>
+static int try_half_stream(const SkinnyArgs& a, int max_tiles, hipStream_t st) {
+  static_assert(StreamCfg<F, RB, 2, 7, D, 2>::kLds <= 80 * 1024, "two work-groups share a CU's LDS");
+  return plan_and_launch<F, EPI, RB, D, 2>(a, 0, max_tiles, st, 2);
 }
 
 // K-steps per wave: prefer a split giving 4..16 waves (balanced reduction
@@ -469,10 +485,13 @@ int ferret_moe_w2_fp8_skinny(const void* h, const float* sh, const void* w, cons
 // fewer waves pay (fewer cross-wave reductions per weight byte): two blocks
 // per unit took 32 experts x 1 row 79 -> 71 us and 256 experts 605 -> 592 us;
 // four blocks on 4 waves of 4 K-steps take 256 experts 593 -> 555 us and
-// 32 experts x 16 rows 82 -> 79 us.
+// 32 experts x 16 rows 82 -> 79 us.  The per-unit kernel, which ran K / 128 of
+// 12 and 6 before, reached 4.2 TB/s of weights: 256 experts x 4 rows, N = 7168,
+// K = 1536 659 -> 425 us (6.5 TB/s); with 15 rows 1079 -> 552, K = 768 634 -> 350.
   a.units_n = N / 16;  // units of the per-unit fallback (RB = 1); try_stream derives its own
   a.pair_tiles = num_pairs >= 10LL * E;
-  const int rc = try_stream<kFP8, kStore, 4, 3, 4>(a, 0, max_tiles, st);
+  int rc = try_stream<kFP8, kStore, 4, 3, 4>(a, 0, max_tiles, st);
+  if (rc == 1) rc = try_half_stream<kFP8, kStore, 4, 3>(a, max_tiles, st);
   if (rc != 1) return rc;
   return launch_skinny<kFP8, kStore, 1>(a, max_tiles, st);
 }

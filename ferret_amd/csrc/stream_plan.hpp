@@ -39,7 +39,8 @@ inline StreamPlan stream_plan(bool silu, int rb, int nw, int N, int K, int tiles
   const int nkb = K >> 7;
   if (nkb % (nw * nsplit) != 0) return p;
   p.ks = nkb / nsplit / nw;
-  if (p.ks != 2 && p.ks != 4 && p.ks != 7 && p.ks != 8) return p;
+  // 3 K-steps per wave: the four-block units of the w2 projection only.
+  if (p.ks != 2 && p.ks != 4 && p.ks != 7 && p.ks != 8 && !(p.ks == 3 && rb == 4)) return p;
   // Past 8 waves a wave has 128 VGPRs: at most 4 K-steps of activations.
   if (nw > 8 && p.ks > 4) return p;
   p.nsplit = nsplit;

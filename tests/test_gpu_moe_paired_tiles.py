@@ -45,7 +45,10 @@ def _weights(E, N, K, padded):
 
 @pytest.mark.parametrize("which,rows,N,K", [
     ("w13", EDGES, 512, 2048), ("w13", EDGES, 256, 4096), ("w13", EDGES, 768, 7168), ("w13", MANY, 256, 2048),
-    ("w2", EDGES, 384, 1024), ("w2", EDGES, 512, 2048), ("w2", EDGES, 128, 3584), ("w2", MANY, 128, 1024)])
+    ("w2", EDGES, 384, 1024), ("w2", EDGES, 512, 2048), ("w2", EDGES, 128, 3584), ("w2", MANY, 128, 1024),
+    # K / 128 of 12 (3 K-steps per wave), then 4, 6 and 14 (two work-groups of 2 waves per CU)
+    ("w2", EDGES, 256, 1536), ("w2", EDGES, 384, 512), ("w2", EDGES, 256, 768), ("w2", EDGES, 128, 1792),
+    ("w2", MANY, 128, 768)])
 def test_two_tiles_per_unit_equal_one(ops, which, rows, N, K):
     from ferret_amd import workloads as W
     E, P = len(rows), sum(rows)

@@ -35,6 +35,11 @@
 // grouped_fp8_gemm_bs<BN,NS> (examples/fp8-group-gemm/v007_dsv3_decode_verified_105.cu:66-335),
 // whose per-K-block epilogue (v002:179-210) this fuses into the main loop.
 #include "common.hpp"
+#include "fp8_mid.hpp"
+
+#include <algorithm>
+
+int ferret_fp8_mid(int tile, const ferret::mid::Args& p, hipStream_t st);
 
 namespace ferret {
 
@@ -588,8 +593,29 @@ static int splitk_splits(int M, int N, int K) {
   return s;
 }
 
+// The small-tile kernel's plan (fp8_mid.hip) for the shapes it takes, else none:
+// one round of work-groups, and K and N where its larger share of token loads
+// costs less than the 128 x 128 tiles' splits.  us against those tiles:
+//   K <= 3072: 4096 x 2048 at 24 / 100 / 256 tokens 7.8 / 12.0 / 13.4 against 8.9 /
+//     15.4 / 20.6; 7168 x 3072 at 256 22.8 against 23.4.  In two rounds it loses
+//     (12288 x 1024 at 256: 19.0 against 12.9).
+//   Larger K, up to 128 tokens while N K <= 22 M: 4096 x 5376 at 100 16.5 against
+//     18.9; 7168 x 4096 at 100 20.5 against 19.5, 4096 x 7168 19.3 against 19.0.
+//   Past 128 tokens while N K <= 11.5 M: 2048 x 5376 at 256 18.4 against 20.1; 2048
+//     x 7168 21.3 against 19.6.
+//   Up to 32 tokens always: 4096 x 7168 at 24 12.3 against 12.7.
+static mid::Plan mid_plan(int M, int N, int K) {
+  const mid::Plan p = mid::plan(M, N, K, SPLITK_TARGET);
+  const long long groups = p.ok ? (long long)p.tok_tiles * (N / (16 * mid::kTiles[p.tile].rt)) * p.splits : 0;
+  const long long nk = (long long)N * K;
+  const bool small = K <= 3072 || nk <= 11500000 || (M <= 128 && nk <= 22100000);
+  return p.ok && (M <= 32 || (small && groups <= SPLITK_TARGET)) ? p : mid::Plan{};
+}
+
+// The larger of the two split-K kernels' partials (which of them runs also
+// depends on the flags).
 size_t ferret_fp8_gemm_workspace(int M, int N, int K) {
-  const int s = splitk_splits(M, N, K);
+  const int s = std::max(splitk_splits(M, N, K), mid_plan(M, N, K).splits);
   return s > 1 ? (size_t)s * M * N * sizeof(float) : 0;
 }
 
@@ -605,9 +631,24 @@ int ferret_fp8_gemm_tiled(const void* a, const float* sa, const void* b, const f
   p.N = N;
   p.K = K;
   p.m_blocks = (M + TB_M - 1) / TB_M;
-  const int splits = splitk_splits(M, N, K);
+  auto reduce_splits = [&](int used) {
+    const size_t n4 = (size_t)M * N / 4;
+    auto* reduce = used == 2 ? splitk_reduce_kernel<2> : used == 4 ? splitk_reduce_kernel<4>
+                 : used == 8 ? splitk_reduce_kernel<8> : splitk_reduce_kernel<0>;
+    hipLaunchKernelGGL(reduce, dim3(512), dim3(256), 0, st, static_cast<const float*>(ws), used, n4,
+                       static_cast<uint16_t*>(c));
+    return (int)hipGetLastError();
+  };
   const size_t need = ferret_fp8_gemm_workspace(M, N, K);
-  if (splits > 1 && ws != nullptr && ws_bytes >= need) {
+  const bool have_ws = ws != nullptr && ws_bytes >= need;
+  const mid::Plan m = f8 ? mid::Plan{} : mid_plan(M, N, K);
+  if (m.ok && (m.splits == 1 || have_ws)) {
+    const mid::Args q{p.a, sa, p.b, sb, p.out, static_cast<float*>(ws), M, N, K, m.splits, m.tok_tiles};
+    const int rc = ferret_fp8_mid(m.tile, q, st);
+    return rc != 0 || m.splits == 1 ? rc : reduce_splits(m.splits);
+  }
+  const int splits = splitk_splits(M, N, K);
+  if (splits > 1 && have_ws) {
     const int nkb = K / TB_K;
     p.k_steps = (nkb + splits - 1) / splits;
     const int used = (nkb + p.k_steps - 1) / p.k_steps;  // splits actually holding K-steps
@@ -616,12 +657,7 @@ int ferret_fp8_gemm_tiled(const void* a, const float* sa, const void* b, const f
     const dim3 grid(p.n_blocks * p.m_blocks, used);
     const int rc = M % TB_M == 0 ? launch_tiled<false, false, SPLITK_WN, true, true, SPLITK_TW>(p, grid, st, f8)
                                  : launch_tiled<false, false, SPLITK_WN, true, false, SPLITK_TW>(p, grid, st, f8);
-    if (rc != 0) return rc;
-    const size_t n4 = (size_t)M * N / 4;
-    auto* reduce = used == 2 ? splitk_reduce_kernel<2> : used == 4 ? splitk_reduce_kernel<4>
-                 : used == 8 ? splitk_reduce_kernel<8> : splitk_reduce_kernel<0>;
-    hipLaunchKernelGGL(reduce, dim3(512), dim3(256), 0, st, p.partial, used, n4, static_cast<uint16_t*>(c));
-    return (int)hipGetLastError();
+    return rc != 0 ? rc : reduce_splits(used);
   }
   // Mid M: where the 256 x 128 grid would fill at most half of the CUs
   // (DSv3 q_b_proj at M = 512: 48 work-groups, each over all of K), the

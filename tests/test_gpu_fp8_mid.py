@@ -1,0 +1,35 @@
+"""The small-tile FP8 product between 16 and 256 tokens: edges of its tiles and K splits.
+
+Against the oracle, with a caller's workspace (its splits) and without (unsplit,
+here or in the larger tiles), at token counts on both sides of every tile size,
+K of one scale block, of an odd number of them and of fewer than the splits.
+"""
+from __future__ import annotations
+
+import pytest
+import torch
+
+from oracle import gemm as G
+from tests.gpu_helpers import assert_gemm_close, bf16_out, codes8, f32
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("M,N,K", [
+    (17, 128, 128), (32, 4096, 384), (33, 256, 2432), (48, 1152, 128), (64, 7168, 640), (65, 128, 3072), (24, 4096, 7168),
+    (96, 384, 1152), (100, 2048, 4224), (128, 4096, 512), (129, 1024, 256), (200, 640, 1664), (256, 256, 3072),
+    (31, 7168, 16384)])
+def test_matches_the_oracle(hip, M, N, K):
+    from ferret_amd import workloads as W
+    print(f"[case] fp8 mid M={M} N={N} K={K}", flush=True)
+    a, sa = W.quant_act_1x128(W.randn((M, K), M + K, "cuda"))
+    b, sb = W.quant_weight_128x128(W.randn((N, K), N, "cuda"))
+    ref = G.fp8_blockscale_gemm(codes8(a), f32(sa), codes8(b), f32(sb))
+    need = int(hip.ferret_workspace_bytes(1, M, N, K, 0))
+    ws = torch.full((max(need, 1),), 0xFF, dtype=torch.uint8, device="cuda")  # NaN partials if any were not written
+    for wp, wn, tag in ((ws.data_ptr(), need, "workspace"), (None, 0, "none")):
+        c = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device="cuda")
+        assert hip.ferret_fp8_gemm_blockscale(a.data_ptr(), sa.data_ptr(), b.data_ptr(), sb.data_ptr(), c.data_ptr(),
+                                              M, N, K, wp, wn, torch.cuda.current_stream().cuda_stream) == 0
+        torch.cuda.synchronize()
+        assert_gemm_close(bf16_out(c), ref, f"fp8 mid {tag}")

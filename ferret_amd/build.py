@@ -22,8 +22,8 @@ CSRC = os.path.join(PKG, "csrc")
 BUILD = os.path.join(PKG, "_build")
 LIB = os.path.join(PKG, "libferret_hip.so")
 NATIVE = os.path.join(PKG, "_native.so")
-SOURCES = ["skinny.hip", "bf16_tiled.hip", "fp8_mid.hip", "fp8_tiled.hip", "fp8_square.hip", "routing.hip", "moe_tail.hip", "ue8m0.hip",
-           "dispatch.hip"]
+SOURCES = ["skinny.hip", "bf16_tiled.hip", "fp8_mid.hip", "int4_moe.hip", "fp8_tiled.hip", "fp8_square.hip",
+           "routing.hip", "moe_tail.hip", "ue8m0.hip", "dispatch.hip"]
 ARCH = "gfx950"
 
 HIPCC_FLAGS = [

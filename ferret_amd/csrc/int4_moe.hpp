@@ -1,0 +1,52 @@
+// LDS layout and range of the two-tile INT4 w13 kernel (int4_moe.hip).  Plain
+// C++17 with no HIP dependency.
+#pragma once
+
+#include <cstdint>
+
+namespace ferret {
+namespace i4 {
+
+constexpr int kWaves = 4;
+constexpr int BW = 2;                                // pairs of 16-row blocks (gate, up) per wave
+constexpr int kItemRows = kWaves * BW * 32;          // weight rows of an item, half of them gate rows
+constexpr int kNS = 3;                               // stages of 128 K
+constexpr int kTB = 2;                               // 16-token tiles per item
+constexpr int kScaleOff = 2 * BW * 1024;             // a wave's weights of a stage, then their scales
+constexpr int kWaveBytes = kScaleOff + BW * 256;
+constexpr int kXOff = kWaves * kWaveBytes;           // a stage's tokens: 32 rows of 256 B
+constexpr int kStage = kXOff + kTB * 16 * 256;
+constexpr int kXLoads = kTB * 16 * 256 / 1024 / kWaves;
+constexpr int kOps = 2 * BW + BW + kXLoads;          // loads per wave and stage
+constexpr int kMaxTiles = 4096;                      // rows of the tile table: 64 words of group-start bits
+constexpr int kBitsOff = kNS * kStage;
+constexpr int kBeforeOff = kBitsOff + kMaxTiles / 8;
+constexpr int kCountOff = kBeforeOff + kMaxTiles / 64 * 4;
+constexpr int kLds = kCountOff + 16;
+static_assert(kLds <= 80 * 1024, "two work-groups share a CU's LDS");
+
+// The rule, for num_pairs routed rows over E experts on ncu CUs (the results
+// are the same bits either way).
+//
+// stream: the persistent stream kernel takes this K.  It is the faster of the
+// two while most experts have one tile; the line lies where enough have two.
+// Rows per expert and time, stream / this kernel (us), N = 1024, K = 7168, 384
+// experts: tiled weights 13: 373 / 359, 14: 385 / 361, 16: 448 / 372 (48 experts
+// of N = 4096: 188 / 188, 196 / 185, 222 / 187; N = 4096, K = 7168, 384 experts at
+// 13: 1385 / 1434); checkpoint layout, whose half cache lines the shorter ring
+// fetches later, 14: 428 / 464, 16: 495 / 481.
+// Other K run on the per-unit kernel, a tile and 16 gate rows per work-group and
+// nothing in flight at its ends: N = 2048, K = 5120, 64 experts 2 / 4 / 8 / 16 rows
+// 108 / 120 / 134 / 199 against 82 / 83 / 84 / 91 us; N = 1024, K = 1024, 128
+// experts 18.8 / 21.6 / 24.7 / 37.1 against 20.5 / 20.2 / 20.1 / 23.3.
+// And the experts' items have to fill both work-groups of every CU: 48 experts
+// of 512 rows are 96 items (18 rows per expert: 48 / 71 us), 16 experts of 2048
+// rows 128 (31 / 43).
+inline bool takes(long long num_pairs, int E, int N, int max_tiles, int ncu, bool stream, bool tiled) {
+  const long long least_rows = stream ? (tiled ? 14 : 16) : 4;
+  return N % kItemRows == 0 && max_tiles <= kMaxTiles && num_pairs >= least_rows * E &&
+         (long long)E * (N / kItemRows) >= 2LL * ncu;
+}
+
+}  // namespace i4
+}  // namespace ferret

@@ -24,8 +24,10 @@
 #include "skinny_kernel.hpp"
 #include "stream_kernel.hpp"
 #include "bf16_tiled.hpp"
+#include "int4_moe.hpp"
 
 int ferret_bf16_tiled(int tile, const ferret::bt::Args& p, hipStream_t st);
+int ferret_int4_moe(const ferret::SkinnyArgs& a, bool tiled, int span, int max_tiles, int ncu, hipStream_t st);
 
 namespace ferret {
 
@@ -121,11 +123,22 @@ static int choose_ks(int nkb, const int* cand, int ncand) {
   return 0;
 }
 
+// K-steps per wave of the per-unit kernel, 0 past its range (K/128 > 128).
+static int unit_steps(int nkb) {
+  static const int cand[] = {4, 7, 8, 2, 1};
+  const int ks = choose_ks(nkb, cand, 5);
+  if (ks != 0) return ks;
+  // No K-step count divides K/128 into <= 16 waves (K/128 = 19, 23, 38, ...):
+  // the smallest of 2, 4, 7, 8 that fits 16 waves, the last wave ragged.
+  for (const int kr : {2, 4, 7, 8})
+    if ((nkb + kr - 1) / kr <= 16) return kr;
+  return 0;
+}
+
 template <int F, int EPI, int RB>
 static int launch_skinny(const SkinnyArgs& a, int ntile_slots, hipStream_t st) {
   const int nkb = a.K >> 7;
-  static const int cand[] = {4, 7, 8, 2, 1};
-  const int ks = choose_ks(nkb, cand, 5);
+  const int ks = unit_steps(nkb);
   const int grid = ntile_slots * a.units_n;
   if (grid <= 0) return FERRET_OK;
   // Prefetch depth kept so a wave stays within 128 VGPRs (16 waves / CU).
@@ -135,20 +148,15 @@ static int launch_skinny(const SkinnyArgs& a, int ntile_slots, hipStream_t st) {
   // spill past 128 VGPRs.
   constexpr int D78 = (F == kFP8 && RB >= 2) ? 2 : DB;
   constexpr int D78R = (F == kFP8 && RB == 1) ? 3 : D78;
-  if (ks == 0) {
-    // No K-step count divides K/128 into <= 16 waves (K/128 = 19, 23, 38, ...):
-    // the smallest of 2, 4, 7, 8 that fits 16 waves, the last wave ragged.
-    for (const int kr : {2, 4, 7, 8}) {
-      const int nw = (nkb + kr - 1) / kr;
-      if (nw > 16) continue;
-      switch (kr) {
-        case 2: return launch_one<F, EPI, RB, 2, 1, true>(a, grid, nw, st);
-        case 4: return launch_one<F, EPI, RB, 4, (DB < 3 ? DB : 3), true>(a, grid, nw, st);
-        case 7: return launch_one<F, EPI, RB, 7, D78R, true>(a, grid, nw, st);
-        case 8: return launch_one<F, EPI, RB, 8, D78R, true>(a, grid, nw, st);
-      }
+  if (ks == 0) return FERRET_ERR_SHAPE;
+  if (nkb % ks != 0) {
+    const int nw = (nkb + ks - 1) / ks;
+    switch (ks) {
+      case 2: return launch_one<F, EPI, RB, 2, 1, true>(a, grid, nw, st);
+      case 4: return launch_one<F, EPI, RB, 4, (DB < 3 ? DB : 3), true>(a, grid, nw, st);
+      case 7: return launch_one<F, EPI, RB, 7, D78R, true>(a, grid, nw, st);
+      case 8: return launch_one<F, EPI, RB, 8, D78R, true>(a, grid, nw, st);
     }
-    return FERRET_ERR_SHAPE;  // K/128 > 128: rejected by every entry point first
   }
   const int nwaves = nkb / ks;
   switch (ks) {
@@ -520,6 +528,16 @@ static int moe_w13_w4a16(const void* x, const int32_t* wq, const void* ws, const
   a.K = K;
   a.units_n = N / 32;
   if (max_tiles <= 0) return FERRET_OK;
+  // The two-tile kernel loads x and the weights as 16-byte chunks, the scales
+  // as words, and stores 8 bytes.  It sums K in the spans of the other kernels'
+  // waves (the stream kernel's eight, or the per-unit kernel's), in their order.
+  const auto bits = [](const void* p) { return reinterpret_cast<uintptr_t>(p); };
+  const int nkb = K >> 7, eighth = nkb % 8 == 0 ? nkb / 8 : 0;
+  const bool stream = (eighth == 2 || eighth == 4 || eighth == 7 || eighth == 8) && (bits(ws) & 15) == 0;
+  const int span = stream ? eighth : unit_steps(nkb);
+  if (span != 0 && ((bits(x) | bits(wq)) & 15) == 0 && (bits(ws) & 3) == 0 && (bits(out) & 7) == 0 &&
+      i4::takes((long long)T * topk, E, N, max_tiles, cu_count(), stream, F == kINT4T))
+    return ferret_int4_moe(a, F == kINT4T, span, max_tiles, cu_count(), st);
   const int rc = try_stream<F, kSilu, 2, 5, 8>(a, 0, max_tiles, st);
   if (rc != 1) return rc;
   return launch_skinny<F, kSilu, 2>(a, max_tiles, st);

@@ -189,11 +189,12 @@ struct StepFrag {
   float sv[RB];
 };
 
-// Groups of up to TB consecutive rows of the tile table with one expert:
-// lead[g] = first table row of group g; returns the group count.  One wave
-// walks the table 64 rows at a time (eight chunks' experts loaded at once).
-template <int TB>
-__device__ __forceinline__ int group_tiles(const int32_t* tiles, int ntiles, int lane, uint16_t* lead) {
+// Groups of up to TB consecutive rows of the tile table with one expert: for
+// every 64 table rows emit(base, firsts, n), the bits of the rows that start a
+// group and the number of groups before them; returns the group count.  One
+// wave walks the table (eight chunks' experts loaded at once).
+template <int TB, class Emit>
+__device__ __forceinline__ int walk_groups(const int32_t* tiles, int ntiles, int lane, Emit&& emit) {
   constexpr int B = 8;
   int n = 0, carry_e = -1, carry_pos = 0;  // the last row walked: its expert, its place in that expert's run
   for (int base0 = 0; base0 < ntiles; base0 += 64 * B) {
@@ -213,13 +214,21 @@ __device__ __forceinline__ int group_tiles(const int32_t* tiles, int ntiles, int
       const int pos = upto != 0 ? lane - (63 - __clzll((long long)upto)) : lane + carry_pos + 1;
       const bool first = base + lane < ntiles && pos % TB == 0;
       const uint64_t firsts = __ballot(first);
-      if (first) lead[n + __popcll(firsts & ((1ull << lane) - 1))] = (uint16_t)(base + lane);
+      emit(base, firsts, n);
       n += __popcll(firsts);
       carry_e = __builtin_amdgcn_readlane(ex[b], 63);
       carry_pos = __builtin_amdgcn_readlane(pos, 63);
     }
   }
   return n;
+}
+
+// lead[g] = first table row of group g.
+template <int TB>
+__device__ __forceinline__ int group_tiles(const int32_t* tiles, int ntiles, int lane, uint16_t* lead) {
+  return walk_groups<TB>(tiles, ntiles, lane, [&](int base, uint64_t firsts, int n) {
+    if (firsts >> lane & 1) lead[n + __popcll(firsts & ((1ull << lane) - 1))] = (uint16_t)(base + lane);
+  });
 }
 
 // tile_slots: dense, the token tiles of M; grouped, the rows of the tile table

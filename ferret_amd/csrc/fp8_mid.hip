@@ -1,6 +1,7 @@
 // FP8 (OCP e4m3) block-scaled product for gfx950 between the decode kernels
 // (16 tokens) and the large tiles: c[M,N] = sum_kb (a_kb . b_kb^T) sa sb for
-// 16 < M <= 256 and the K where it beats the split-K tiles of fp8_tiled.hip.
+// 16 < M <= 256 and the K where it beats the split-K tiles of fp8_tiled.hip, and
+// past 256 tokens where its work-groups fit one round.
 //
 // These shapes are a few microseconds of loads between fixed costs: a launch,
 // the first stage, the epilogue and, where K is split, 13 MB of fp32 partials

@@ -64,5 +64,28 @@ inline Plan plan(int M, int N, int K, int ncu) {
   return best;
 }
 
+// Past 256 tokens, where K is not split: the tile with the least estimated time
+// of those whose work-groups fit one round.  64 x 128 only from K = 512 on: its
+// epilogue outlasts one or two stages (3072 x 128 at 583 tokens 5.2 us against
+// 4.5 with 128 x 128 tiles; 4096 x 384 at 400 6.8 / 6.6, 4096 x 512 at 368 6.7 /
+// 7.5).
+inline Plan unsplit_plan(int M, int N, int K, int ncu) {
+  Plan best;
+  if (M <= 256 || N <= 0 || N % 128 != 0 || K <= 0 || K % 128 != 0 || K > 16384) return best;
+  double best_us = 0;
+  for (int i = 0; i < kNumTiles; ++i) {
+    const Tile& t = kTiles[i];
+    const long long tok_tiles = ((long long)M + 16 * t.tt - 1) / (16 * t.tt);
+    if (tok_tiles * (N / (16 * t.rt)) > ncu || (K < 512 && t.rt * t.tt > 16)) continue;
+    const double us = (K / 128 + 1) / 2 * t.us;
+    if (best.ok && us >= best_us) continue;
+    best_us = us;
+    best.ok = true;
+    best.tile = i;
+    best.tok_tiles = (int)tok_tiles;
+  }
+  return best;
+}
+
 }  // namespace mid
 }  // namespace ferret

@@ -604,7 +604,14 @@ static int splitk_splits(int M, int N, int K) {
 //   Past 128 tokens while N K <= 11.5 M: 2048 x 5376 at 256 18.4 against 20.1; 2048
 //     x 7168 21.3 against 19.6.
 //   Up to 32 tokens always: 4096 x 7168 at 24 12.3 against 12.7.
+// Past 256 tokens there is no split, and 128 x 128 tiles that leave CUs idle take
+// 0.95 us for each 128 of K whatever their number: one round of smaller tiles is
+// the shorter.  4096 x 7168 at 320 / 512 tokens 45.6 / 47.5 against 53.8 / 54.9;
+// 2048 x 4096 at 512 / 1000 21.3 / 29.5 against 32.3 / 33.4; 1536 x 7168 at 320 24.8
+// against 55.1; geometric mean 1.48 over 70 shapes.  In two rounds they lose (7168
+// x 2048 at 320: 28.6 against 18.4).
 static mid::Plan mid_plan(int M, int N, int K) {
+  if (M > 256) return mid::unsplit_plan(M, N, K, SPLITK_TARGET);
   const mid::Plan p = mid::plan(M, N, K, SPLITK_TARGET);
   const long long groups = p.ok ? (long long)p.tok_tiles * (N / (16 * mid::kTiles[p.tile].rt)) * p.splits : 0;
   const long long nk = (long long)N * K;
@@ -660,7 +667,7 @@ int ferret_fp8_gemm_tiled(const void* a, const float* sa, const void* b, const f
     return rc != 0 ? rc : reduce_splits(used);
   }
   // Mid M: where the 256 x 128 grid would fill at most half of the CUs
-  // (DSv3 q_b_proj at M = 512: 48 work-groups, each over all of K), the
+  // (DSv3 q_b_proj at M = 1000: 96 work-groups, each over all of K), the
   // 128 x 128 tiles of the split-K configuration double it while it still
   // fits one round, and store bf16 directly.
   const int t256 = ((N + 255) / 256) * p.m_blocks;

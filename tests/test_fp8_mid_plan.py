@@ -34,6 +34,18 @@ int main() {
         }
         if (at != nkb) BAD("cover");
       }
+  for (int M : {1, 256, 257, 320, 511, 512, 513, 1000, 4096, 16384, 16385, 1000000})
+    for (int nkb : {1, 3, 4, 19, 56, 128, 129})
+      for (int N : {128, 384, 1024, 4096, 7168, 16384, 24576}) {
+        const Plan p = unsplit_plan(M, N, nkb * 128, 256);
+        const bool fits = M > 256 && nkb <= 128 && (long long)((M + 63) / 64) * (N / 64) <= 256;
+        if (fits && !p.ok) BAD("not taken");
+        if (!p.ok) continue;
+        if (M <= 256 || nkb > 128 || p.splits != 1) BAD("taken");
+        const Tile& t = kTiles[p.tile];
+        if (p.tok_tiles * t.tt * 16 < M || (p.tok_tiles - 1) * t.tt * 16 >= M) BAD("tokens");
+        if (p.tok_tiles * (N / (16 * t.rt)) > 256) BAD("rounds");
+      }
   std::printf("plans %lld\n", plans);
   return 0;
 }

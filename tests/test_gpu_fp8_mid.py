@@ -1,4 +1,4 @@
-"""The small-tile FP8 product between 16 and 256 tokens: edges of its tiles and K splits.
+"""The small-tile FP8 product past 16 tokens: edges of its tiles and K splits.
 
 Against the oracle, with a caller's workspace (its splits) and without (unsplit,
 here or in the larger tiles), at token counts on both sides of every tile size,
@@ -18,7 +18,10 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K", [
     (17, 128, 128), (32, 4096, 384), (33, 256, 2432), (48, 1152, 128), (64, 7168, 640), (65, 128, 3072), (24, 4096, 7168),
     (96, 384, 1152), (100, 2048, 4224), (128, 4096, 512), (129, 1024, 256), (200, 640, 1664), (256, 256, 3072),
-    (31, 7168, 16384)])
+    (31, 7168, 16384),
+    # past 256 tokens, never split: every tile, odd block counts, the last shape of one round and the first past it
+    (257, 1024, 128), (300, 256, 2432), (1313, 128, 384), (490, 1024, 1152), (512, 2048, 640), (1024, 2048, 512),
+    (1025, 2048, 512), (269, 1536, 16384)])
 def test_matches_the_oracle(hip, M, N, K):
     from ferret_amd import workloads as W
     print(f"[case] fp8 mid M={M} N={N} K={K}", flush=True)

@@ -39,13 +39,17 @@ static_assert(kLds <= 80 * 1024, "two work-groups share a CU's LDS");
 // nothing in flight at its ends: N = 2048, K = 5120, 64 experts 2 / 4 / 8 / 16 rows
 // 108 / 120 / 134 / 199 against 82 / 83 / 84 / 91 us; N = 1024, K = 1024, 128
 // experts 18.8 / 21.6 / 24.7 / 37.1 against 20.5 / 20.2 / 20.1 / 23.3.
-// And the experts' items have to fill both work-groups of every CU: 48 experts
-// of 512 rows are 96 items (18 rows per expert: 48 / 71 us), 16 experts of 2048
-// rows 128 (31 / 43).
+// And the items have to fill the CUs: both work-groups of each if every expert
+// had one, or three quarters of them by the 32-row groups there must be.  48
+// experts of 512 rows are 96 items of one group (18 rows per expert: 48 / 71 us),
+// 16 experts of 2048 rows 128 (31 / 43); by groups, 16 experts of 2048 rows, K =
+// 4096 reach the line at 96 rows per expert (24 / 64 / 96 / 256 rows: 32 / 73 / 99 /
+// 244 against 46 / 69 / 71 / 167), 48 experts of 512 at 128 (48 / 64 / 128 rows: 79 /
+// 96 / 176 against 80 / 82 / 127).
 inline bool takes(long long num_pairs, int E, int N, int max_tiles, int ncu, bool stream, bool tiled) {
-  const long long least_rows = stream ? (tiled ? 14 : 16) : 4;
+  const long long least_rows = stream ? (tiled ? 14 : 16) : 4, nb = N / kItemRows;
   return N % kItemRows == 0 && max_tiles <= kMaxTiles && num_pairs >= least_rows * E &&
-         (long long)E * (N / kItemRows) >= 2LL * ncu;
+         (E * nb >= 2LL * ncu || num_pairs / 32 * nb >= ncu + ncu / 2);
 }
 
 }  // namespace i4

@@ -33,14 +33,15 @@ def ops(hip):
 @pytest.mark.parametrize("E,N,K", [(128, 1024, 128), (128, 1024, 256), (64, 2048, 384),  # as few stages as the ring
                                    (600, 256, 2048), (130, 1024, 2048),                  # a long table; the stream kernel's K
                                    (64, 2048, 2432),                                     # ragged last span
-                                   (33, 4096, 7168)])
+                                   (33, 4096, 7168),
+                                   (8, 1024, 2048)])                                     # few experts of many rows
 def test_two_tiles_equal_one(ops, E, N, K):
-    rows = _rows(E)
+    rows = _rows(E) if E > 8 else [n * 24 for n in EDGES[:8]]
     P = sum(rows)
     streams = K in (2048, 7168)  # the K of the stream kernel: 14 (tiled) or 16 rows per expert, else 4
     padded = P // (14 if streams else 4) + 1
     print(f"[case] int4 two tiles E={E} P={P} N={N} K={K}", flush=True)
-    assert 16 * E <= P and E * (N // 256) >= 512 and padded <= 1024
+    assert 16 * E <= P and padded <= 1024 and (E * (N // 256) >= 512 or P // 32 * (N // 256) >= 384)
     ids = np.concatenate([np.full(n, e, dtype=np.int32) for e, n in enumerate(rows)])
     np.random.default_rng(E).shuffle(ids)
     ids = torch.from_numpy(ids.reshape(-1, 1)).cuda()

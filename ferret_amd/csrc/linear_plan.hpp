@@ -1,0 +1,75 @@
+// Dispatch rules of the bf16 linear (ferret_linear_bf16 in skinny.hip): which
+// kernel takes a shape, its K split and its workspace.  Plain C++17 without HIP,
+// so that CPU tests compile the rules themselves.
+#pragma once
+
+#include <cstddef>
+#include <cstdint>
+
+#include "bf16_tiled.hpp"
+#include "stream_plan.hpp"
+
+namespace ferret {
+namespace lin {
+
+// K splits of the bf16 stream kernel for y = x.W^T: 1 when a work-group per CU
+// is already evenly loaded (>= 90 % of the 256 CUs' share), else the split with
+// the best balance whose K-steps per wave (of 8) the kernel instantiates.
+// Measured reason: 384 row units (QKV) leave half the CUs with one unit and
+// half with two; K = 12288 (Down) needs 12 K-steps per wave, more activation
+// registers than a wave has.
+inline int stream_splits(int M, int N, int K, int ncu) {
+  const int nkb = K / 128;
+  const long long units = (long long)((M + 15) / 16) * (N / 16);
+  auto ks_ok = [](int ks) { return ks == 2 || ks == 4 || ks == 7 || ks == 8; };
+  auto balance = [&](int s) {
+    const long long items = units * s;
+    const long long per = (items + ncu - 1) / ncu;
+    return (double)items / (double)(per * ncu);
+  };
+  if (nkb % 8 == 0 && ks_ok(nkb / 8) && balance(1) >= 0.9) return 1;
+  int best = 1;
+  double best_b = -1.0;
+  for (int s = 2; s <= 8; ++s) {
+    if (nkb % (8 * s) != 0 || !ks_ok(nkb / (8 * s))) continue;
+    const double b = balance(s);
+    if (b > best_b + 1e-9) { best = s; best_b = b; }
+  }
+  return best;
+}
+
+// The LDS-tiled kernel's plan for the shapes it takes, else none.
+//   * Past 16 tokens: it streams the weights once for all of them, the stream
+//     and per-unit kernels once per 16 (4096 x 12288 at 17 tokens 20.5 against
+//     36.2 us, 24576 x 4096 at 32 32.7 against 45.5, 6144 x 4096 at 32 14.1
+//     against 14.7).
+//   * Up to 16 tokens where the stream kernel does not take K (K / 128 not 2, 4,
+//     7 or 8 per wave; 1536 x 9984: 11.2 against the per-unit kernel's 17.4 us
+//     at one token, 12.1 against 23.4 at 16; 16000 x 1280 9.0 against 10.9 and
+//     9.2 against 14.7).
+//   * Not where the whole product is a few microseconds: a split's second launch
+//     and the ring's fill cost 2-3 us more than the other kernels spend.  In
+//     16-token tiles x N x K the line lies at 2^25 against the stream kernel (4
+//     tiles of 2048 x 2048, 2^24: 9.7 against 7.0 us; 2 of 4096 x 4096, 2^25:
+//     10.4 against 13.9) and at 10 * 2^20 against the per-unit one (2 tiles of
+//     4096 x 640: 5.8 against 5.3; 4: 6.7 against 7.7).
+inline bt::Plan tiled_plan(int M, int N, int K, int ncu) {
+  const bool stream = stream_plan(false, 1, 8, N, K, 1, false, stream_splits(M, N, K, ncu), ncu).ok ||
+                      (N / 16 >= 4 * ncu && stream_plan(false, 1, 4, N, K, 1, false, 1, ncu).ok);
+  const long long work = (long long)((M + 15) / 16) * N * K;
+  if ((stream && M <= 16) || work < (stream ? 32LL : 10LL) << 20) return bt::Plan{};
+  return bt::plan(M, N, K, ncu);
+}
+
+// The tiled kernel copies x and the weights global -> LDS 16 bytes at a time,
+// reads the residual and stores y 8 bytes at a time, and keeps its partials in
+// 16-byte pieces.  Tensors off these bounds (a view that starts inside a buffer)
+// keep the kernels of 16 tokens, which load x through registers and store single
+// elements.
+inline bool tiled_aligned(const void* x, const void* w, const void* residual, const void* y, const void* ws) {
+  const auto bits = [](const void* p) { return reinterpret_cast<uintptr_t>(p); };
+  return ((bits(x) | bits(w) | bits(ws)) & 15) == 0 && ((bits(residual) | bits(y)) & 7) == 0;
+}
+
+}  // namespace lin
+}  // namespace ferret

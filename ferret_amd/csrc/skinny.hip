@@ -23,7 +23,7 @@
 // the INT4 w13 contract (tasks/kimi-moe-w13-int4-grouped-gemm.yaml:68-95,150-167).
 #include "skinny_kernel.hpp"
 #include "stream_kernel.hpp"
-#include "bf16_tiled.hpp"
+#include "linear_plan.hpp"
 #include "int4_moe.hpp"
 
 int ferret_bf16_tiled(int tile, const ferret::bt::Args& p, hipStream_t st);
@@ -225,68 +225,17 @@ static int launch_bf16_tiled(const bt::Plan& plan, const SkinnyArgs& a, int n0, 
   return launch_splitk_reduce(p.partial, p.splits, p.M, p.N, p.ldo, p.residual, p.out, st);
 }
 
-// K splits of the bf16 stream kernel for y = x.W^T: 1 when a work-group per CU
-// is already evenly loaded (>= 90 % of the 256 CUs' share), else the split with
-// the best balance whose K-steps per wave (of 8) the kernel instantiates.
-// Measured reason: 384 row units (QKV) leave half the CUs with one unit and
-// half with two; K = 12288 (Down) needs 12 K-steps per wave, more activation
-// registers than a wave has.
-static int linear_splits(int M, int N, int K) {
-  const int nkb = K / 128;
-  const long long units = (long long)((M + 15) / 16) * (N / 16);
-  const int ncu = cu_count();
-  auto ks_ok = [](int ks) { return ks == 2 || ks == 4 || ks == 7 || ks == 8; };
-  auto balance = [&](int s) {
-    const long long items = units * s;
-    const long long per = (items + ncu - 1) / ncu;
-    return (double)items / (double)(per * ncu);
-  };
-  if (nkb % 8 == 0 && ks_ok(nkb / 8) && balance(1) >= 0.9) return 1;
-  int best = 1;
-  double best_b = -1.0;
-  for (int s = 2; s <= 8; ++s) {
-    if (nkb % (8 * s) != 0 || !ks_ok(nkb / (8 * s))) continue;
-    const double b = balance(s);
-    if (b > best_b + 1e-9) { best = s; best_b = b; }
-  }
-  return best;
-}
-
-// The LDS-tiled kernel's plan for the shapes it takes, else none.
-//   * Past 16 tokens: it streams the weights once for all of them, the stream
-//     and per-unit kernels once per 16 (4096 x 12288 at 17 tokens 20.5 against
-//     36.2 us, 24576 x 4096 at 32 32.7 against 45.5, 6144 x 4096 at 32 14.1
-//     against 14.7).
-//   * Up to 16 tokens where the stream kernel does not take K (K / 128 not 2, 4,
-//     7 or 8 per wave; 1536 x 9984: 11.2 against the per-unit kernel's 17.4 us
-//     at one token, 12.1 against 23.4 at 16; 16000 x 1280 9.0 against 10.9 and
-//     9.2 against 14.7).
-//   * Not where the whole product is a few microseconds: a split's second launch
-//     and the ring's fill cost 2-3 us more than the other kernels spend.  In
-//     16-token tiles x N x K the line lies at 2^25 against the stream kernel (4
-//     tiles of 2048 x 2048, 2^24: 9.7 against 7.0 us; 2 of 4096 x 4096, 2^25:
-//     10.4 against 13.9) and at 10 * 2^20 against the per-unit one (2 tiles of
-//     4096 x 640: 5.8 against 5.3; 4: 6.7 against 7.7).
-static bt::Plan tiled_plan(int M, int N, int K) {
-  const int ncu = cu_count();
-  const bool stream = stream_plan(false, 1, 8, N, K, 1, false, linear_splits(M, N, K), ncu).ok ||
-                      (N / 16 >= 4 * ncu && stream_plan(false, 1, 4, N, K, 1, false, 1, ncu).ok);
-  const long long work = (long long)((M + 15) / 16) * N * K;
-  if ((stream && M <= 16) || work < (stream ? 32LL : 10LL) << 20) return bt::Plan{};
-  return bt::plan(M, N, K, ncu);
-}
-
 }  // namespace ferret
 
 using namespace ferret;
 
 static size_t linear_workspace(const bt::Plan& tiled, int M, int N, int K) {
-  const int s = tiled.ok ? tiled.splits : linear_splits(M, N, K);
+  const int s = tiled.ok ? tiled.splits : lin::stream_splits(M, N, K, cu_count());
   return s > 1 ? (size_t)s * M * N * sizeof(float) : 0;
 }
 
 size_t ferret_linear_bf16_workspace(int M, int N, int K) {
-  return linear_workspace(tiled_plan(M, N, K), M, N, K);
+  return linear_workspace(lin::tiled_plan(M, N, K, cu_count()), M, N, K);
 }
 
 extern "C" int ferret_linear_bf16(const void* x, const void* w, const void* residual, void* y, int M,
@@ -304,10 +253,12 @@ extern "C" int ferret_linear_bf16(const void* x, const void* w, const void* resi
   a.N = N;
   a.K = K;
   a.units_n = N / 16;
-  const bt::Plan tiled = tiled_plan(M, N, K);
+  const bt::Plan tiled = lin::tiled_plan(M, N, K, cu_count());
   const size_t need = linear_workspace(tiled, M, N, K);
-  if (tiled.ok && (need == 0 || (ws != nullptr && ws_bytes >= need))) return launch_bf16_tiled(tiled, a, 0, N, ws, st);
-  const int splits = tiled.ok ? 1 : linear_splits(M, N, K);
+  if (tiled.ok && (need == 0 || (ws != nullptr && ws_bytes >= need)) &&
+      lin::tiled_aligned(x, w, residual, y, need == 0 ? nullptr : ws))
+    return launch_bf16_tiled(tiled, a, 0, N, ws, st);
+  const int splits = tiled.ok ? 1 : lin::stream_splits(M, N, K, cu_count());
   if (splits > 1 && ws != nullptr && ws_bytes >= need && (M * (long long)N) % 4 == 0) {
     a.partial = static_cast<float*>(ws);
     a.ksplit = splits;
@@ -376,13 +327,14 @@ extern "C" int ferret_linear_bf16_noalloc(const void* x, const void* w, const vo
   FERRET_REQUIRE(x && w && y, FERRET_ERR_NULL);
   FERRET_REQUIRE(M >= 1 && N >= 16 && K >= 128, FERRET_ERR_SHAPE);
   FERRET_REQUIRE(N % 16 == 0 && K % 128 == 0 && K / 128 <= 128, FERRET_ERR_SHAPE);
-  const int splits = linear_splits(M, N, K);
+  const int splits = lin::stream_splits(M, N, K, cu_count());
   FERRET_REQUIRE(splits <= 1 || (size_t)splits * M * N * sizeof(float) <= kNoAllocScratchBytes, FERRET_ERR_WORKSPACE);
-  const bt::Plan tiled = tiled_plan(M, N, K);
+  const bt::Plan tiled = lin::tiled_plan(M, N, K, cu_count());
   const size_t need = linear_workspace(tiled, M, N, K);
   void* ws = nullptr;
   if (need > 0) FERRET_HIP_CHECK(scratch_address(&ws));
-  if (!tiled.ok || need <= kNoAllocScratchBytes) return ferret_linear_bf16(x, w, residual, y, M, N, K, ws, need, stream);
+  if (!tiled.ok || need <= kNoAllocScratchBytes || !lin::tiled_aligned(x, w, residual, y, nullptr))
+    return ferret_linear_bf16(x, w, residual, y, M, N, K, ws, std::min(need, kNoAllocScratchBytes), stream);
   // Partials larger than the array: the same plan over runs of whole row tiles
   // whose partials fit (each output's sums are those of one launch).
   SkinnyArgs a{};

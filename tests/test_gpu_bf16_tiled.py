@@ -63,3 +63,31 @@ def test_allocation_free_entry_gives_the_same_bits(hip, M, N, K, res):
 def ops(hip):
     from ferret_amd import ops as O
     return O
+
+
+def _at(t, elements):
+    """t's values in a contiguous tensor that starts `elements` into its allocation."""
+    buf = torch.zeros(t.numel() + elements, dtype=t.dtype, device=t.device)
+    v = buf[elements:].view(t.shape)
+    v.copy_(t)
+    return v
+
+
+@pytest.mark.parametrize("M,N,K", [(40, 1552, 1280), (64, 6144, 4096), (7, 1536, 9984)])
+@pytest.mark.parametrize("which", ["x", "residual", "out"])
+def test_unaligned_tensors_keep_the_earlier_kernels(ops, hip, M, N, K, which):
+    """Views that start inside a buffer: x 8 bytes past a 16-byte bound, residual or y 2 bytes past one."""
+    print(f"[case] bf16 linear unaligned {which} M={M} N={N} K={K}", flush=True)
+    x, w, r = _inputs(M, N, K, True)
+    y = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device="cuda")
+    ref = G.linear_bf16(bits16(x), bits16(w), bits16(r))
+    x, r, y = (_at(t, 0 if which != name else 4 if name == "x" else 1)
+               for t, name in ((x, "x"), (r, "residual"), (y, "out")))
+    ops.linear_bf16(x, w, r, out=y)
+    torch.cuda.synchronize()
+    assert_gemm_close(bf16_out(y), ref, f"unaligned {which}")
+    y.fill_(float("nan"))
+    assert hip.ferret_linear_bf16_noalloc(x.data_ptr(), w.data_ptr(), r.data_ptr(), y.data_ptr(), M, N, K,
+                                          torch.cuda.current_stream().cuda_stream) == 0
+    torch.cuda.synchronize()
+    assert_gemm_close(bf16_out(y), ref, f"unaligned {which}, allocation-free entry")

@@ -1,0 +1,36 @@
+"""CPU checks of the bf16 linear's dispatch rules (ferret_amd/csrc/linear_plan.hpp), compiled with g++."""
+import os
+import shutil
+import subprocess
+
+import pytest
+
+CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "ferret_amd", "csrc")
+
+
+def run_rules(tmp_path, body):
+    """Compile `body` (the statements of main) against the rules, run it and return its output."""
+    gxx = shutil.which("g++")
+    if gxx is None:
+        pytest.skip("g++ not available")
+    src, exe = tmp_path / "route.cpp", tmp_path / "route"
+    src.write_text('#include <cstdio>\n#include <initializer_list>\n#include "linear_plan.hpp"\n'
+                   "using namespace ferret;\n#define CHECK(c) do { if (!(c)) { std::printf(\"%s\\n\", #c); return 1; } } "
+                   "while (0)\nint main() {\n" + body + "\n  return 0;\n}\n")
+    subprocess.run([gxx, "-std=c++17", "-O2", "-I", CSRC, str(src), "-o", str(exe)], check=True)
+    res = subprocess.run([str(exe)], capture_output=True, text=True, timeout=300)
+    assert res.returncode == 0, res.stdout
+    return res.stdout
+
+
+def test_tiled_kernel_takes_aligned_tensors_only(tmp_path):
+    run_rules(tmp_path, r"""
+  alignas(64) static char buf[5][128];
+  for (int which = 0; which < 5; ++which)  // x, w, residual, y, workspace
+    for (int off = 0; off <= 32; off += 2) {
+      char* p[5];
+      for (int i = 0; i < 5; ++i) p[i] = buf[i] + (i == which ? off : 0);
+      const int bound = which == 2 || which == 3 ? 8 : 16;
+      CHECK(lin::tiled_aligned(p[0], p[1], p[2], p[3], p[4]) == (off % bound == 0));
+    }
+  CHECK(lin::tiled_aligned(buf[0], buf[1], nullptr, buf[3], nullptr));""")

@@ -25,6 +25,7 @@
 #include "stream_kernel.hpp"
 #include "linear_plan.hpp"
 #include "int4_moe.hpp"
+#include "moe_plan.hpp"
 
 int ferret_bf16_tiled(int tile, const ferret::bt::Args& p, hipStream_t st);
 int ferret_int4_moe(const ferret::SkinnyArgs& a, bool tiled, int span, int max_tiles, int ncu, hipStream_t st);
@@ -450,9 +451,11 @@ int ferret_moe_w2_fp8_skinny(const void* h, const float* sh, const void* w, cons
 // K = 1536 659 -> 425 us (6.5 TB/s); with 15 rows 1079 -> 552, K = 768 634 -> 350.
   a.units_n = N / 16;  // units of the per-unit fallback (RB = 1); try_stream derives its own
   a.pair_tiles = num_pairs >= 10LL * E;
-  int rc = try_stream<kFP8, kStore, 4, 3, 4>(a, 0, max_tiles, st);
-  if (rc == 1) rc = try_half_stream<kFP8, kStore, 4, 3>(a, max_tiles, st);
-  if (rc != 1) return rc;
+  if (moe::w2_streams(K >> 7, w)) {
+    int rc = try_stream<kFP8, kStore, 4, 3, 4>(a, 0, max_tiles, st);
+    if (rc == 1) rc = try_half_stream<kFP8, kStore, 4, 3>(a, max_tiles, st);
+    if (rc != 1) return rc;
+  }
   return launch_skinny<kFP8, kStore, 1>(a, max_tiles, st);
 }
 

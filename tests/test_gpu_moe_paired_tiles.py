@@ -69,3 +69,21 @@ def test_two_tiles_per_unit_equal_one(ops, which, rows, N, K):
         oracle = G.moe_w13_fp8 if which == "w13" else G.moe_w2_fp8
         ref = oracle(codes8(x), f32(sx), codes8(w[:E]), f32(sw[:E]), ids.cpu().numpy())
         assert_gemm_close(bf16_out(got), ref, f"{which} N={N} K={K}")
+
+
+@pytest.mark.parametrize("K", [1536, 512, 768, 1792])
+def test_w2_weights_off_a_16_byte_bound(ops, K):
+    """K / 128 = 12, 4, 6 and 14: weights that start 8 bytes into a buffer keep the per-unit kernel."""
+    from ferret_amd import workloads as W
+    E, N, P = 6, 256, 40
+    print(f"[case] w2 unaligned weights K={K}", flush=True)
+    ids = torch.arange(P, device="cuda", dtype=torch.int32).remainder(E).view(-1, 1).contiguous()
+    x, sx = W.quant_act_1x128(W.randn((P, K), 11, "cuda"))
+    w, sw = _weights(E, N, K, E)
+    buf = torch.zeros(w.numel() + 8, dtype=torch.uint8, device="cuda")
+    off = buf[8:].view(w.shape)
+    off.copy_(w.view(torch.uint8))
+    got = ops.moe_w2_fp8(x, sx, off, sw, ops.moe_permute(ids, E, 16))
+    torch.cuda.synchronize()
+    ref = G.moe_w2_fp8(codes8(x), f32(sx), codes8(w), f32(sw), ids.cpu().numpy())
+    assert_gemm_close(bf16_out(got), ref, f"w2 unaligned K={K}")

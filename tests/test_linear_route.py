@@ -8,13 +8,13 @@ import pytest
 CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "ferret_amd", "csrc")
 
 
-def run_rules(tmp_path, body):
-    """Compile `body` (the statements of main) against the rules, run it and return its output."""
+def run_rules(tmp_path, body, header="linear_plan.hpp"):
+    """Compile `body` (the statements of main) against a header of rules, run it and return its output."""
     gxx = shutil.which("g++")
     if gxx is None:
         pytest.skip("g++ not available")
     src, exe = tmp_path / "route.cpp", tmp_path / "route"
-    src.write_text('#include <cstdio>\n#include <initializer_list>\n#include "linear_plan.hpp"\n'
+    src.write_text('#include <cstdio>\n#include <initializer_list>\n#include "' + header + '"\n'
                    "using namespace ferret;\n#define CHECK(c) do { if (!(c)) { std::printf(\"%s\\n\", #c); return 1; } } "
                    "while (0)\nint main() {\n" + body + "\n  return 0;\n}\n")
     subprocess.run([gxx, "-std=c++17", "-O2", "-I", CSRC, str(src), "-o", str(exe)], check=True)

@@ -19,6 +19,7 @@ struct Args {
   int tok_tiles;             // token tiles
   int rt0;                   // row tiles before this launch's first (its place in the K rotation)
   bool nt;                   // stream the weights past the caches
+  int rot_rows;              // serial form: rows of the plan's tiles (a place in the K rotation each)
 };
 
 // The tiles the kernel is built for: rt x 16 weight rows by tt x 16 tokens,

@@ -71,5 +71,11 @@ inline bool tiled_aligned(const void* x, const void* w, const void* residual, co
   return ((bits(x) | bits(w) | bits(ws)) & 15) == 0 && ((bits(residual) | bits(y)) & 7) == 0;
 }
 
+// Whether the allocation-free entry takes its partials from the library's one
+// array, so that calls which overlap race: only where the 16-token kernels split
+// K.  Any other call may overlap with all of them, and be captured into a graph
+// before the array's address is known.
+inline bool noalloc_shares_array(int M, int N, int K, int ncu) { return stream_splits(M, N, K, ncu) > 1; }
+
 }  // namespace lin
 }  // namespace ferret

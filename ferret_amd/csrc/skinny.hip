@@ -28,6 +28,7 @@
 #include "moe_plan.hpp"
 
 int ferret_bf16_tiled(int tile, const ferret::bt::Args& p, hipStream_t st);
+int ferret_bf16_tiled_serial(int tile, ferret::bt::Args p, hipStream_t st);
 int ferret_int4_moe(const ferret::SkinnyArgs& a, bool tiled, int span, int max_tiles, int ncu, hipStream_t st);
 
 namespace ferret {
@@ -201,21 +202,27 @@ static int launch_splitk_reduce(const float* partial, int S, int M, int N, int l
   return (int)hipGetLastError();
 }
 
-// The LDS-tiled product over weight rows [n0, n0 + n) by `plan`, partials in ws.
-static int launch_bf16_tiled(const bt::Plan& plan, const SkinnyArgs& a, int n0, int n, void* ws, hipStream_t st) {
-  const bt::Tile& t = bt::kTiles[plan.tile];
+// Arguments of the LDS-tiled product over weight rows [n0, n0 + n) by `plan`.
+static bt::Args bf16_tiled_args(const bt::Plan& plan, const SkinnyArgs& a, int n0, int n) {
   bt::Args p{};
   p.w = a.w + (size_t)n0 * a.K * 2;
   p.x = a.x;
   p.residual = a.residual ? a.residual + n0 : nullptr;
   p.out = a.out + n0;
-  p.partial = static_cast<float*>(ws);
   p.M = a.M;
   p.N = n;
   p.K = a.K;
   p.ldo = a.N;
   p.splits = plan.splits;
   p.tok_tiles = plan.tok_tiles;
+  return p;
+}
+
+// The LDS-tiled product over weight rows [n0, n0 + n) by `plan`, partials in ws.
+static int launch_bf16_tiled(const bt::Plan& plan, const SkinnyArgs& a, int n0, int n, void* ws, hipStream_t st) {
+  const bt::Tile& t = bt::kTiles[plan.tile];
+  bt::Args p = bf16_tiled_args(plan, a, n0, n);
+  p.partial = static_cast<float*>(ws);
   p.rt0 = n0 / (16 * t.rt);
   // Weights that only one work-group reads: past the caches (24576 x 4096 at 64
   // tokens 37.3 -> 34.0 us, 4096 x 12288 at 32 22.0 -> 20.3); beside the tokens
@@ -224,6 +231,11 @@ static int launch_bf16_tiled(const bt::Plan& plan, const SkinnyArgs& a, int n0, 
   const int rc = ferret_bf16_tiled(plan.tile, p, st);
   if (rc != 0 || plan.splits == 1) return rc;
   return launch_splitk_reduce(p.partial, p.splits, p.M, p.N, p.ldo, p.residual, p.out, st);
+}
+
+// The same result from one launch with no partials.
+static int launch_bf16_tiled_serial(const bt::Plan& plan, const SkinnyArgs& a, hipStream_t st) {
+  return ferret_bf16_tiled_serial(plan.tile, bf16_tiled_args(plan, a, 0, a.N), st);
 }
 
 }  // namespace ferret
@@ -291,7 +303,9 @@ extern "C" int ferret_linear_bf16(const void* x, const void* w, const void* resi
 // (hipGetSymbolAddress, with that device current) and only that address is
 // handed to kernels.  Calls that overlap on one GPU share the array and race;
 // every split writes all of its partials before the reduce reads them, so
-// nothing needs clearing between calls.
+// nothing needs clearing between calls.  Only shapes that the 16-token kernels
+// split use it (lin::noalloc_shares_array); the tiled kernel's splits of all
+// others run in its serial form.
 constexpr size_t kNoAllocScratchBytes = 4u << 20;
 static __device__ __align__(256) uint8_t scratch[kNoAllocScratchBytes];
 static std::atomic<void*> g_scratch_ptr[64];
@@ -332,12 +346,6 @@ extern "C" int ferret_linear_bf16_noalloc(const void* x, const void* w, const vo
   FERRET_REQUIRE(splits <= 1 || (size_t)splits * M * N * sizeof(float) <= kNoAllocScratchBytes, FERRET_ERR_WORKSPACE);
   const bt::Plan tiled = lin::tiled_plan(M, N, K, cu_count());
   const size_t need = linear_workspace(tiled, M, N, K);
-  void* ws = nullptr;
-  if (need > 0) FERRET_HIP_CHECK(scratch_address(&ws));
-  if (!tiled.ok || need <= kNoAllocScratchBytes || !lin::tiled_aligned(x, w, residual, y, nullptr))
-    return ferret_linear_bf16(x, w, residual, y, M, N, K, ws, std::min(need, kNoAllocScratchBytes), stream);
-  // Partials larger than the array: the same plan over runs of whole row tiles
-  // whose partials fit (each output's sums are those of one launch).
   SkinnyArgs a{};
   a.w = static_cast<const uint8_t*>(w);
   a.x = static_cast<const uint8_t*>(x);
@@ -346,6 +354,17 @@ extern "C" int ferret_linear_bf16_noalloc(const void* x, const void* w, const vo
   a.M = M;
   a.N = N;
   a.K = K;
+  const bool aligned = lin::tiled_aligned(x, w, residual, y, nullptr);
+  if (!lin::noalloc_shares_array(M, N, K, cu_count())) {
+    if (tiled.ok && tiled.splits > 1 && aligned) return launch_bf16_tiled_serial(tiled, a, (hipStream_t)stream);
+    return ferret_linear_bf16(x, w, residual, y, M, N, K, nullptr, 0, stream);
+  }
+  void* ws = nullptr;
+  FERRET_HIP_CHECK(scratch_address(&ws));
+  if (!tiled.ok || need <= kNoAllocScratchBytes || !aligned)
+    return ferret_linear_bf16(x, w, residual, y, M, N, K, ws, std::min(need, kNoAllocScratchBytes), stream);
+  // Partials larger than the array: the same plan over runs of whole row tiles
+  // whose partials fit (each output's sums are those of one launch).
   const int tile_rows = 16 * bt::kTiles[tiled.tile].rt;
   const int rows = (int)(kNoAllocScratchBytes / ((size_t)tiled.splits * M * sizeof(float))) / tile_rows * tile_rows;
   for (int n0 = 0; n0 < N; n0 += rows) {

@@ -68,17 +68,19 @@ int ferret_linear_bf16(const void* x, const void* w, const void* residual, void*
  * ferret_linear_bf16 without a workspace argument and without any allocation:
  * no counterpart in the reference.  For callers that cannot allocate (code
  * under HIP graph capture, tight serving loops, harnesses that forbid
- * hipMalloc).  Shapes that run split-K take their fp32 partials from a
- * library-owned device array of ferret_linear_bf16_noalloc_max_bytes()
- * (4 MiB) per GPU; a shape whose partials by 16-token tiles need more (M = 100,
- * N = 4096, K = 12288) is rejected with FERRET_ERR_WORKSPACE, and one that
- * needs more only because it takes all tokens at once (M > 16) runs in several
- * ranges of weight rows.  The result is bit-identical to ferret_linear_bf16
- * with a workspace.  Calls that overlap on
- * one GPU (different streams or threads) share the array and race: serialise
+ * hipMalloc).  Shapes whose 16-token tiles run split-K (K/128 a multiple of 8
+ * that is uneven over the CUs, e.g. N = 6144, K = 4096 at M <= 16, or K = 12288)
+ * take their fp32 partials from a library-owned device array of
+ * ferret_linear_bf16_noalloc_max_bytes() (4 MiB) per GPU; one whose partials by
+ * 16-token tiles need more (M = 100, N = 4096, K = 12288) is rejected with
+ * FERRET_ERR_WORKSPACE, and one that needs more only because it takes all tokens
+ * at once (M > 16) runs in several ranges of weight rows.  All other shapes use
+ * no memory but their arguments.  The result is bit-identical to
+ * ferret_linear_bf16 with a workspace.  Calls that use the array and overlap on
+ * one GPU (different streams or threads) share it and race: serialise
  * them.  The array's address is looked up once per device, by the first call
- * of ferret_linear_bf16_noalloc_max_bytes or of this entry point on it: make
- * one of them on each device before capturing this entry point into a graph.
+ * of ferret_linear_bf16_noalloc_max_bytes or of this entry point on such a
+ * shape: make one of them on each device before capturing one into a graph.
  */
 int ferret_linear_bf16_noalloc(const void* x, const void* w, const void* residual, void* y, int M,
                                int N, int K, void* stream);

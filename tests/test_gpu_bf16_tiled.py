@@ -91,3 +91,52 @@ def test_unaligned_tensors_keep_the_earlier_kernels(ops, hip, M, N, K, which):
                                           torch.cuda.current_stream().cuda_stream) == 0
     torch.cuda.synchronize()
     assert_gemm_close(bf16_out(y), ref, f"unaligned {which}, allocation-free entry")
+
+
+def _workspace_bits(hip, x, w, r, M, N, K):
+    need = int(hip.ferret_workspace_bytes(0, M, N, K, 0))
+    ws = torch.full((need,), 0xFF, dtype=torch.uint8, device="cuda")
+    y = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device="cuda")
+    assert need > 0 and hip.ferret_linear_bf16(
+        x.data_ptr(), w.data_ptr(), r.data_ptr() if r is not None else None, y.data_ptr(), M, N, K, ws.data_ptr(),
+        need, torch.cuda.current_stream().cuda_stream) == 0
+    return y
+
+
+# One shape per tile and token-tile count that splits K where the 16-token kernels did not (these run without the
+# library's array), then shapes whose 16-token split uses it: partials that fit, and row ranges.
+@pytest.mark.parametrize("M,N,K,res", [
+    (5, 4096, 2560, True), (5, 4320, 2432, False), (20, 1008, 5248, True), (20, 4272, 1280, False),
+    (33, 1440, 2432, True), (33, 3280, 1664, False), (50, 1584, 1664, True), (50, 4224, 1280, False),
+    (70, 1824, 1152, True), (100, 592, 2560, False), (70, 3360, 1280, True), (100, 1648, 1280, False),
+    (100, 2144, 1408, True), (97, 2720, 1152, True), (200, 1008, 2816, False), (5, 6368, 1664, True),
+    (200, 2704, 1792, False),
+    (48, 4096, 12288, True), (64, 4096, 12288, True), (80, 4096, 12288, False)])
+def test_allocation_free_entry_gives_the_same_bits_on_every_tile(hip, M, N, K, res):
+    print(f"[case] bf16 tiled noalloc M={M} N={N} K={K} res={res}", flush=True)
+    x, w, r = _inputs(M, N, K, res)
+    want = _workspace_bits(hip, x, w, r, M, N, K)
+    hip.ferret_linear_bf16_noalloc_max_bytes()
+    y = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device="cuda")
+    assert hip.ferret_linear_bf16_noalloc(x.data_ptr(), w.data_ptr(), r.data_ptr() if res else None, y.data_ptr(),
+                                          M, N, K, torch.cuda.current_stream().cuda_stream) == 0
+    torch.cuda.synchronize()
+    assert torch.equal(y.view(torch.int16), want.view(torch.int16))
+
+
+def test_allocation_free_calls_without_a_16_token_split_may_overlap(hip):
+    """Two streams at once, shapes whose 16-token split is one: no memory is shared."""
+    shapes = [(64, 4096, 4096), (8, 1536, 9984)]
+    print("[case] bf16 tiled noalloc on two streams", flush=True)
+    ins = [_inputs(*s, False) for s in shapes]
+    want = [_workspace_bits(hip, x, w, None, *s) for s, (x, w, _) in zip(shapes, ins)]
+    outs = [[torch.empty((M, N), dtype=torch.bfloat16, device="cuda") for _ in range(20)] for M, N, _ in shapes]
+    streams = [torch.cuda.Stream() for _ in shapes]
+    torch.cuda.synchronize()
+    for i in range(20):
+        for (M, N, K), (x, w, _), out, st in zip(shapes, ins, outs, streams):
+            assert hip.ferret_linear_bf16_noalloc(x.data_ptr(), w.data_ptr(), None, out[i].data_ptr(), M, N, K,
+                                                  st.cuda_stream) == 0
+    torch.cuda.synchronize()
+    for out, y in zip(outs, want):
+        assert all(torch.equal(o.view(torch.int16), y.view(torch.int16)) for o in out)

@@ -34,3 +34,15 @@ def test_tiled_kernel_takes_aligned_tensors_only(tmp_path):
       CHECK(lin::tiled_aligned(p[0], p[1], p[2], p[3], p[4]) == (off % bound == 0));
     }
   CHECK(lin::tiled_aligned(buf[0], buf[1], nullptr, buf[3], nullptr));""")
+
+
+def test_allocation_free_entry_shares_its_array_only_where_16_token_tiles_split(tmp_path):
+    """Shapes that ran unsplit before the tiled kernel took them must not write to the library's one array."""
+    run_rules(tmp_path, r"""
+  const int shared[][3] = {{16, 6144, 4096}, {5, 4096, 12288}, {48, 4096, 12288}, {16, 1536, 4096}};
+  for (auto& s : shared) CHECK(lin::noalloc_shares_array(s[0], s[1], s[2], 256));
+  const int own[][3] = {{64, 4096, 4096}, {20, 4096, 4096}, {64, 6144, 4096}, {8, 1536, 9984}, {100, 2144, 1408}};
+  for (auto& s : own) {
+    const bt::Plan p = lin::tiled_plan(s[0], s[1], s[2], 256);
+    CHECK(p.ok && p.splits > 1 && !lin::noalloc_shares_array(s[0], s[1], s[2], 256));
+  }""")

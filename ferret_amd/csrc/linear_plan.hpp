@@ -71,6 +71,33 @@ inline bool tiled_aligned(const void* x, const void* w, const void* residual, co
   return ((bits(x) | bits(w) | bits(ws)) & 15) == 0 && ((bits(residual) | bits(y)) & 7) == 0;
 }
 
+// fp32 partials of S splits.
+inline size_t partial_bytes(int S, int M, int N) { return S > 1 ? (size_t)S * M * N * sizeof(float) : 0; }
+
+// What a call runs: the LDS-tiled kernel by `tiled` where that is ok, else the
+// 16-token kernels with K split by `splits`.
+struct Route {
+  bt::Plan tiled;
+  int splits = 1;
+};
+
+// Each kernel asks for its own partials only: a workspace that a caller sized for
+// the 16-token split (4096 x 12288 at 48 tokens: 3 splits, the tiled plan has 4)
+// still holds that split, and tensors off the tiled kernel's bounds still take it.
+inline Route route(int M, int N, int K, int ncu, const void* x, const void* w, const void* residual, const void* y,
+                   const void* ws, size_t ws_bytes) {
+  if (ws == nullptr) ws_bytes = 0;
+  Route r;
+  r.tiled = tiled_plan(M, N, K, ncu);
+  const size_t need = partial_bytes(r.tiled.splits, M, N);
+  if (need > ws_bytes || !tiled_aligned(x, w, residual, y, need == 0 ? nullptr : ws)) r.tiled.ok = false;
+  if (!r.tiled.ok) {
+    const int s = stream_splits(M, N, K, ncu);
+    if (partial_bytes(s, M, N) <= ws_bytes) r.splits = s;
+  }
+  return r;
+}
+
 // Whether the allocation-free entry takes its partials from the library's one
 // array, so that calls which overlap race: only where the 16-token kernels split
 // K.  Any other call may overlap with all of them, and be captured into a graph

@@ -243,8 +243,7 @@ static int launch_bf16_tiled_serial(const bt::Plan& plan, const SkinnyArgs& a, h
 using namespace ferret;
 
 static size_t linear_workspace(const bt::Plan& tiled, int M, int N, int K) {
-  const int s = tiled.ok ? tiled.splits : lin::stream_splits(M, N, K, cu_count());
-  return s > 1 ? (size_t)s * M * N * sizeof(float) : 0;
+  return lin::partial_bytes(tiled.ok ? tiled.splits : lin::stream_splits(M, N, K, cu_count()), M, N);
 }
 
 size_t ferret_linear_bf16_workspace(int M, int N, int K) {
@@ -266,13 +265,10 @@ extern "C" int ferret_linear_bf16(const void* x, const void* w, const void* resi
   a.N = N;
   a.K = K;
   a.units_n = N / 16;
-  const bt::Plan tiled = lin::tiled_plan(M, N, K, cu_count());
-  const size_t need = linear_workspace(tiled, M, N, K);
-  if (tiled.ok && (need == 0 || (ws != nullptr && ws_bytes >= need)) &&
-      lin::tiled_aligned(x, w, residual, y, need == 0 ? nullptr : ws))
-    return launch_bf16_tiled(tiled, a, 0, N, ws, st);
-  const int splits = tiled.ok ? 1 : lin::stream_splits(M, N, K, cu_count());
-  if (splits > 1 && ws != nullptr && ws_bytes >= need && (M * (long long)N) % 4 == 0) {
+  const lin::Route route = lin::route(M, N, K, cu_count(), x, w, residual, y, ws, ws_bytes);
+  if (route.tiled.ok) return launch_bf16_tiled(route.tiled, a, 0, N, ws, st);
+  const int splits = route.splits;
+  if (splits > 1) {
     a.partial = static_cast<float*>(ws);
     a.ksplit = splits;
     const int rc = try_stream<kBF16, kStore, 1, 3, 8>(a, (M + 15) / 16, 0, st);
@@ -362,7 +358,7 @@ extern "C" int ferret_linear_bf16_noalloc(const void* x, const void* w, const vo
   void* ws = nullptr;
   FERRET_HIP_CHECK(scratch_address(&ws));
   if (!tiled.ok || need <= kNoAllocScratchBytes || !aligned)
-    return ferret_linear_bf16(x, w, residual, y, M, N, K, ws, std::min(need, kNoAllocScratchBytes), stream);
+    return ferret_linear_bf16(x, w, residual, y, M, N, K, ws, kNoAllocScratchBytes, stream);
   // Partials larger than the array: the same plan over runs of whole row tiles
   // whose partials fit (each output's sums are those of one launch).
   const int tile_rows = 16 * bt::kTiles[tiled.tile].rt;

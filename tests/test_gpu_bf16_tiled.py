@@ -93,6 +93,23 @@ def test_unaligned_tensors_keep_the_earlier_kernels(ops, hip, M, N, K, which):
     assert_gemm_close(bf16_out(y), ref, f"unaligned {which}, allocation-free entry")
 
 
+@pytest.mark.parametrize("M,N,K,splits", [(48, 4096, 12288, 3), (64, 1536, 12288, 6)])
+def test_workspace_of_the_16_token_split(hip, M, N, K, splits):
+    """Smaller than the tiled plan's partials: the 16-token kernels split K in it, and write no byte past it."""
+    size = splits * M * N * 4
+    print(f"[case] bf16 linear small workspace M={M} N={N} K={K} bytes {size}", flush=True)
+    assert size < hip.ferret_workspace_bytes(0, M, N, K, 0)
+    x, w, r = _inputs(M, N, K, True)
+    ws = torch.full((size + 4096,), 0xFF, dtype=torch.uint8, device="cuda")
+    y = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device="cuda")
+    assert hip.ferret_linear_bf16(x.data_ptr(), w.data_ptr(), r.data_ptr(), y.data_ptr(), M, N, K, ws.data_ptr(), size,
+                                  torch.cuda.current_stream().cuda_stream) == 0
+    torch.cuda.synchronize()
+    assert_gemm_close(bf16_out(y), G.linear_bf16(bits16(x), bits16(w), bits16(r)), "small workspace")
+    assert bool((ws[size:] == 0xFF).all())
+    assert not bool((ws[:size].view(torch.int32) == -1).any())   # every partial was written
+
+
 def _workspace_bits(hip, x, w, r, M, N, K):
     need = int(hip.ferret_workspace_bytes(0, M, N, K, 0))
     ws = torch.full((need,), 0xFF, dtype=torch.uint8, device="cuda")

@@ -46,3 +46,27 @@ def test_allocation_free_entry_shares_its_array_only_where_16_token_tiles_split(
     const bt::Plan p = lin::tiled_plan(s[0], s[1], s[2], 256);
     CHECK(p.ok && p.splits > 1 && !lin::noalloc_shares_array(s[0], s[1], s[2], 256));
   }""")
+
+
+def test_each_kernel_asks_for_its_own_partials(tmp_path):
+    """A workspace of the 16-token split, or tensors off the tiled kernel's bounds, keep that split."""
+    run_rules(tmp_path, r"""
+  alignas(64) static char b[5][64];
+  const auto route = [](const int* s, size_t bytes, int off = 0, bool ws = true) {
+    return lin::route(s[0], s[1], s[2], 256, b[0] + off, b[1], b[2], b[3], ws ? b[4] : nullptr, bytes);
+  };
+  // M, N, K, splits of the tiled plan and of the 16-token kernels
+  const int shapes[][5] = {{48, 4096, 12288, 4, 3}, {64, 1536, 12288, 8, 6}, {24, 6144, 4096, 4, 1}, {16, 4096, 12288, 0, 3}};
+  for (auto& s : shapes) {
+    const size_t one = (size_t)s[0] * s[1] * 4, tiled = one * s[3], units = s[4] > 1 ? one * s[4] : 0;
+    if (s[3]) {
+      CHECK(route(s, tiled).tiled.ok && route(s, tiled).tiled.splits == s[3]);
+      CHECK(!route(s, tiled - 1).tiled.ok && route(s, tiled - 1).splits == s[4]);
+      CHECK(!route(s, tiled, 8).tiled.ok && route(s, tiled, 8).splits == s[4]);
+    }
+    CHECK(!route(s, units).tiled.ok && route(s, units).splits == s[4]);
+    if (units) CHECK(route(s, units - 1).splits == 1);
+    CHECK(!route(s, 1 << 30, 0, false).tiled.ok && route(s, 1 << 30, 0, false).splits == 1);
+  }
+  const int unsplit[3] = {64, 24576, 4096};  // needs no workspace and looks at none
+  CHECK(route(unsplit, 0, 0, false).tiled.ok && lin::route(64, 24576, 4096, 256, b[0], b[1], b[2], b[3], b[4] + 1, 8).tiled.ok);""")

@@ -35,9 +35,7 @@
 // grouped_fp8_gemm_bs<BN,NS> (examples/fp8-group-gemm/v007_dsv3_decode_verified_105.cu:66-335),
 // whose per-K-block epilogue (v002:179-210) this fuses into the main loop.
 #include "common.hpp"
-#include "fp8_mid.hpp"
-
-#include <algorithm>
+#include "fp8_plan.hpp"
 
 int ferret_fp8_mid(int tile, const ferret::mid::Args& p, hipStream_t st);
 
@@ -574,60 +572,15 @@ static int launch_tiled(const TiledArgs& p, dim3 grid, hipStream_t st, bool f8) 
             : launch_tiled_one<SILU, GROUPED, WN, SPLIT, FULL, false, TW>(p, grid, st);
 }
 
-// Split-K plan for small M: 128 x 128 tiles (8 waves) over K ranges, the
-// number of splits the largest power of two whose grid still fits the 256 CUs
-// in one round (one 97.5-KB work-group per CU): a grid of 448 at
-// 128 x 7168 x 2048 ran in two rounds, 26.5 us against 15.7 us with 224.
-// At 128 x 4096 x 7168 (256 work-groups) this beat 64 x 128 and 256 x 128
-// tiles and two work-groups per CU (28 us vs 29-36 us).  Returns the number
-// of splits (1 = no split-K).
+// The 128 x 128 tiles of 8 waves that split K for small M (fp8_plan.hpp).
 constexpr int SPLITK_WN = 2;         // 128 x 128 tiles
 constexpr int SPLITK_TW = 4;         // of 8 waves (64 x 32 each, two per SIMD)
-constexpr int SPLITK_TARGET = 256;   // work-groups the split grid may not exceed (one per CU)
-static int splitk_splits(int M, int N, int K) {
-  if (M > 256 || N % (64 * SPLITK_WN) != 0) return 1;
-  const int tiles = (N / (64 * SPLITK_WN)) * ((M + TB_M - 1) / TB_M);
-  const int nkb = K / TB_K;
-  int s = 1;
-  while (tiles * s * 2 <= SPLITK_TARGET && s * 2 <= nkb / 2) s *= 2;
-  return s;
-}
+static_assert(TB_M == 128 && TB_K == 128 && 64 * SPLITK_WN == 128, "the tiles fp8_plan.hpp counts");
 
-// The small-tile kernel's plan (fp8_mid.hip) for the shapes it takes, else none:
-// one round of work-groups, and K and N where its larger share of token loads
-// costs less than the 128 x 128 tiles' splits.  us against those tiles:
-//   K <= 3072: 4096 x 2048 at 24 / 100 / 256 tokens 7.8 / 12.0 / 13.4 against 8.9 /
-//     15.4 / 20.6; 7168 x 3072 at 256 22.8 against 23.4.  In two rounds it loses
-//     (12288 x 1024 at 256: 19.0 against 12.9).
-//   Larger K, up to 128 tokens while N K <= 22 M: 4096 x 5376 at 100 16.5 against
-//     18.9; 7168 x 4096 at 100 20.5 against 19.5, 4096 x 7168 19.3 against 19.0.
-//   Past 128 tokens while N K <= 11.5 M: 2048 x 5376 at 256 18.4 against 20.1; 2048
-//     x 7168 21.3 against 19.6.
-//   Up to 32 tokens always: 4096 x 7168 at 24 12.3 against 12.7.
-// Past 256 tokens there is no split, and 128 x 128 tiles that leave CUs idle take
-// 0.95 us for each 128 of K whatever their number: one round of smaller tiles is
-// the shorter.  4096 x 7168 at 320 / 512 tokens 45.6 / 47.5 against 53.8 / 54.9;
-// 2048 x 4096 at 512 / 1000 21.3 / 29.5 against 32.3 / 33.4; 1536 x 7168 at 320 24.8
-// against 55.1; geometric mean 1.48 over 70 shapes.  In two rounds they lose (7168
-// x 2048 at 320: 28.6 against 18.4).
-static mid::Plan mid_plan(int M, int N, int K) {
-  if (M > 256) return mid::unsplit_plan(M, N, K, SPLITK_TARGET);
-  const mid::Plan p = mid::plan(M, N, K, SPLITK_TARGET);
-  const long long groups = p.ok ? (long long)p.tok_tiles * (N / (16 * mid::kTiles[p.tile].rt)) * p.splits : 0;
-  const long long nk = (long long)N * K;
-  const bool small = K <= 3072 || nk <= 11500000 || (M <= 128 && nk <= 22100000);
-  return p.ok && (M <= 32 || (small && groups <= SPLITK_TARGET)) ? p : mid::Plan{};
-}
-
-// The larger of the two split-K kernels' partials (which of them runs also
-// depends on the flags).
-size_t ferret_fp8_gemm_workspace(int M, int N, int K) {
-  const int s = std::max(splitk_splits(M, N, K), mid_plan(M, N, K).splits);
-  return s > 1 ? (size_t)s * M * N * sizeof(float) : 0;
-}
+size_t ferret_fp8_gemm_workspace(int M, int N, int K) { return f8::workspace(M, N, K); }
 
 int ferret_fp8_gemm_tiled(const void* a, const float* sa, const void* b, const float* sb, void* c, int M,
-                          int N, int K, void* ws, size_t ws_bytes, bool f8, hipStream_t st) {
+                          int N, int K, void* ws, size_t ws_bytes, bool e4m3, hipStream_t st) {
   TiledArgs p{};
   p.a = static_cast<const uint8_t*>(a);
   p.sa = sa;
@@ -646,24 +599,23 @@ int ferret_fp8_gemm_tiled(const void* a, const float* sa, const void* b, const f
                        static_cast<uint16_t*>(c));
     return (int)hipGetLastError();
   };
-  const size_t need = ferret_fp8_gemm_workspace(M, N, K);
-  const bool have_ws = ws != nullptr && ws_bytes >= need;
-  const mid::Plan m = f8 ? mid::Plan{} : mid_plan(M, N, K);
-  if (m.ok && (m.splits == 1 || have_ws)) {
+  const f8::Route route = f8::route(M, N, K, e4m3, ws != nullptr ? ws_bytes : 0);
+  if (route.mid.ok) {
+    const mid::Plan& m = route.mid;
     const mid::Args q{p.a, sa, p.b, sb, p.out, static_cast<float*>(ws), M, N, K, m.splits, m.tok_tiles};
     const int rc = ferret_fp8_mid(m.tile, q, st);
     return rc != 0 || m.splits == 1 ? rc : reduce_splits(m.splits);
   }
-  const int splits = splitk_splits(M, N, K);
-  if (splits > 1 && have_ws) {
+  const int splits = route.splits;
+  if (splits > 1) {
     const int nkb = K / TB_K;
     p.k_steps = (nkb + splits - 1) / splits;
     const int used = (nkb + p.k_steps - 1) / p.k_steps;  // splits actually holding K-steps
     p.partial = static_cast<float*>(ws);
     p.n_blocks = N / (64 * SPLITK_WN);
     const dim3 grid(p.n_blocks * p.m_blocks, used);
-    const int rc = M % TB_M == 0 ? launch_tiled<false, false, SPLITK_WN, true, true, SPLITK_TW>(p, grid, st, f8)
-                                 : launch_tiled<false, false, SPLITK_WN, true, false, SPLITK_TW>(p, grid, st, f8);
+    const int rc = M % TB_M == 0 ? launch_tiled<false, false, SPLITK_WN, true, true, SPLITK_TW>(p, grid, st, e4m3)
+                                 : launch_tiled<false, false, SPLITK_WN, true, false, SPLITK_TW>(p, grid, st, e4m3);
     return rc != 0 ? rc : reduce_splits(used);
   }
   // Mid M: where the 256 x 128 grid would fill at most half of the CUs
@@ -672,16 +624,16 @@ int ferret_fp8_gemm_tiled(const void* a, const float* sa, const void* b, const f
   // fits one round, and store bf16 directly.
   const int t256 = ((N + 255) / 256) * p.m_blocks;
   const int t128 = (N / (64 * SPLITK_WN)) * p.m_blocks;
-  if (2 * t256 <= SPLITK_TARGET && t128 <= SPLITK_TARGET) {
+  if (2 * t256 <= f8::kRound && t128 <= f8::kRound) {
     p.n_blocks = N / (64 * SPLITK_WN);
-    if (M % TB_M == 0) return launch_tiled<false, false, SPLITK_WN, false, true, SPLITK_TW>(p, dim3(t128), st, f8);
-    return launch_tiled<false, false, SPLITK_WN, false, false, SPLITK_TW>(p, dim3(t128), st, f8);
+    if (M % TB_M == 0) return launch_tiled<false, false, SPLITK_WN, false, true, SPLITK_TW>(p, dim3(t128), st, e4m3);
+    return launch_tiled<false, false, SPLITK_WN, false, false, SPLITK_TW>(p, dim3(t128), st, e4m3);
   }
   // Dense tiles: with every token tile full (M % 128 == 0) the kernel skips
   // the per-wave count of occupied 16-token sub-tiles.
   p.n_blocks = (N + 255) / 256;
-  if (M % TB_M == 0) return launch_tiled<false, false, 4, false, true>(p, dim3(p.n_blocks * p.m_blocks), st, f8);
-  return launch_tiled<false, false, 4, false, false>(p, dim3(p.n_blocks * p.m_blocks), st, f8);
+  if (M % TB_M == 0) return launch_tiled<false, false, 4, false, true>(p, dim3(p.n_blocks * p.m_blocks), st, e4m3);
+  return launch_tiled<false, false, 4, false, false>(p, dim3(p.n_blocks * p.m_blocks), st, e4m3);
 }
 
 int ferret_moe_w13_fp8_tiled(const void* x, const float* sx, const void* w, const float* sw,

@@ -12,6 +12,7 @@
 // on the same stream.  Shapes of the 256 x 256 kernel skip it: that kernel
 // reads the packed bytes and scales each operand exactly while widening it.
 #include "common.hpp"
+#include "fp8_plan.hpp"
 
 namespace ferret {
 
@@ -43,21 +44,11 @@ __global__ __launch_bounds__(256) void ue8m0_decode_kernel(const uint32_t* __res
   }
 }
 
-constexpr size_t kUe8m0Align = 256;
-inline size_t align_up(size_t v) { return (v + kUe8m0Align - 1) / kUe8m0Align * kUe8m0Align; }
-
 }  // namespace ferret
 
 using namespace ferret;
 
-size_t ferret_fp8_gemm_workspace(int M, int N, int K);
-
-// Workspace of ferret_fp8_gemm_ue8m0: the decoded scales, then the GEMM's own.
-size_t ferret_fp8_gemm_ue8m0_workspace(int M, int N, int K) {
-  const size_t nk = (size_t)K / 128, nbk = ((size_t)N + 127) / 128;
-  const size_t gemm = M > 16 ? ferret_fp8_gemm_workspace(M, N, K) : 0;
-  return align_up((size_t)M * nk * 4) + align_up(nbk * nk * 4) + gemm;
-}
+size_t ferret_fp8_gemm_ue8m0_workspace(int M, int N, int K) { return f8::ue8m0_workspace(M, N, K); }
 
 extern "C" int ferret_fp8_gemm_blockscale(const void* a, const float* sa, const void* b, const float* sb, void* c,
                                           int M, int N, int K, void* ws, size_t ws_bytes, void* stream);
@@ -71,8 +62,7 @@ extern "C" int ferret_fp8_gemm_ue8m0(const void* a, const uint32_t* sfa, const v
   FERRET_REQUIRE(M >= 1 && N >= 16 && K >= 128 && N % 16 == 0 && K % 128 == 0 && K / 128 <= 128,
                  FERRET_ERR_SHAPE);
   FERRET_REQUIRE(M <= 16 || N % 128 == 0, FERRET_ERR_SHAPE);
-  const size_t need = ferret_fp8_gemm_ue8m0_workspace(M, N, K);
-  FERRET_REQUIRE(ws != nullptr && ws_bytes >= need, FERRET_ERR_WORKSPACE);
+  FERRET_REQUIRE(ws != nullptr && ws_bytes >= f8::ue8m0_least_workspace(M, N, K), FERRET_ERR_WORKSPACE);
   // Shapes of the 256 x 256 kernel take the packed bytes directly: each
   // power-of-two scale is applied while its operand is widened to bf16 (no
   // decode pass, no running rescale).
@@ -81,9 +71,9 @@ extern "C" int ferret_fp8_gemm_ue8m0(const void* a, const uint32_t* sfa, const v
   const int nk = K / 128, nbk = (N + 127) / 128;
   uint8_t* base = static_cast<uint8_t*>(ws);
   float* sa = reinterpret_cast<float*>(base);
-  float* sb = reinterpret_cast<float*>(base + align_up((size_t)M * nk * 4));
-  uint8_t* gemm_ws = base + align_up((size_t)M * nk * 4) + align_up((size_t)nbk * nk * 4);
-  const size_t gemm_bytes = need - (size_t)(gemm_ws - base);
+  float* sb = reinterpret_cast<float*>(base + f8::align_up((size_t)M * nk * 4));
+  uint8_t* gemm_ws = base + f8::ue8m0_scale_bytes(M, N, K);
+  const size_t gemm_bytes = ws_bytes - f8::ue8m0_scale_bytes(M, N, K);
   const hipStream_t st = (hipStream_t)stream;
   const long long total = (long long)M * nk + (long long)nbk * nk;
   const int grid = (int)((total + 255) / 256 < 1024 ? (total + 255) / 256 : 1024);

@@ -98,8 +98,9 @@ size_t ferret_linear_bf16_noalloc_max_bytes(void);
  * Requirements: M >= 1, N % 16 == 0, K % 128 == 0 (N % 128 == 0 when M > 16).
  * For 16 < M <= 256 the product runs split-K when `ws` holds at least
  * ferret_workspace_bytes(1, M, N, K, 0) bytes (fp32 partials, summed in a fixed
- * order: deterministic); with ws == NULL the same result comes from the
- * non-split kernel (slower at these shapes).
+ * order: deterministic); a smaller one is used as far as it holds the partials
+ * of the 128 x 128 tiles (fewer splits), and with ws == NULL the same result
+ * comes from the non-split kernel (slower at these shapes).
  */
 int ferret_fp8_gemm_blockscale(const void* a, const float* sa, const void* b, const float* sb,
                                void* c, int M, int N, int K, void* ws, size_t ws_bytes,
@@ -118,9 +119,9 @@ int ferret_fp8_gemm_blockscale(const void* a, const float* sa, const void* b, co
  * :478-484), so c[m,n] = sum_kb (sum_{k in kb} a[m,k] b[n,k]) * 2^(ea-127) *
  * 2^(eb-127), the reference's oracle ref_bs (:486-505).  a e4m3 [M,K],
  * b e4m3 [N,K], c bf16 [M,N]; requirements as ferret_fp8_gemm_blockscale.
- * `ws` is required: at least ferret_workspace_bytes(5, M, N, K, 0) bytes (the
- * scales decoded to fp32, then the GEMM's split-K partials); a smaller one
- * returns FERRET_ERR_WORKSPACE.
+ * `ws` is required: ferret_workspace_bytes(5, M, N, K, 0) bytes (the scales
+ * decoded to fp32, then the GEMM's split-K partials); one too small for the
+ * scales and the partials of the 128 x 128 tiles returns FERRET_ERR_WORKSPACE.
  */
 int ferret_fp8_gemm_ue8m0(const void* a, const uint32_t* sfa, const void* b, const uint32_t* sfb, void* c,
                           int M, int N, int K, void* ws, size_t ws_bytes, void* stream);

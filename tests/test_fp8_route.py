@@ -1,0 +1,26 @@
+"""CPU checks of the FP8 product's dispatch rules past 16 tokens (ferret_amd/csrc/fp8_plan.hpp), compiled with g++."""
+from tests.test_linear_route import run_rules
+
+
+def test_each_kernel_asks_for_its_own_partials(tmp_path):
+    """A workspace of the 128 x 128 tiles' split keeps that split where the small tiles' is larger, with either
+    matrix instruction, and the UE8M0 entry takes it."""
+    run_rules(tmp_path, r"""
+  // M, N, K, splits of the small tiles and of the 128 x 128 tiles
+  const int shapes[][5] = {{17, 128, 1408, 8, 4}, {100, 512, 1664, 8, 4}, {200, 640, 1664, 4, 4}, {128, 4096, 512, 1, 2}};
+  for (auto& s : shapes) {
+    const int M = s[0], N = s[1], K = s[2];
+    const size_t small = f8::partial_bytes(s[3], M, N), tiles = f8::partial_bytes(s[4], M, N);
+    const size_t need = small > tiles ? small : tiles, sc = f8::ue8m0_scale_bytes(M, N, K);
+    CHECK(f8::mid_plan(M, N, K).splits == s[3] && f8::tile_splits(M, N, K) == s[4] && f8::workspace(M, N, K) == need);
+    CHECK(f8::route(M, N, K, false, need).mid.splits == s[3] && f8::route(M, N, K, false, need).mid.ok);
+    CHECK(!f8::route(M, N, K, true, tiles).mid.ok && f8::route(M, N, K, true, tiles).splits == s[4]);
+    CHECK(f8::route(M, N, K, true, tiles - 1).splits == 1);
+    if (small > tiles) {
+      CHECK(!f8::route(M, N, K, false, small - 1).mid.ok && f8::route(M, N, K, false, tiles).splits == s[4]);
+      CHECK(f8::route(M, N, K, false, tiles - 1).splits == 1 && f8::route(M, N, K, false, 0).splits == 1);
+    }
+    CHECK(f8::ue8m0_workspace(M, N, K) == sc + need && f8::ue8m0_least_workspace(M, N, K) == sc + tiles);
+  }
+  for (int M : {17, 100, 256}) for (int N : {128, 4096, 24576}) for (int K : {128, 1536, 7168, 16384})
+    CHECK(f8::ue8m0_least_workspace(M, N, K) <= f8::ue8m0_workspace(M, N, K));""", "fp8_plan.hpp")

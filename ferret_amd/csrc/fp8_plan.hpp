@@ -38,7 +38,11 @@ inline int tile_splits(int M, int N, int K) {
 //     18.9; 7168 x 4096 at 100 20.5 against 19.5, 4096 x 7168 19.3 against 19.0.
 //   Past 128 tokens while N K <= 11.5 M: 2048 x 5376 at 256 18.4 against 20.1; 2048
 //     x 7168 21.3 against 19.6.
-//   Up to 32 tokens always: 4096 x 7168 at 24 12.3 against 12.7.
+//   Up to 32 tokens any K: 4096 x 7168 at 24 12.3 against 12.7.  In more than one
+//     round it loses there too (34944 x 1024 at 23 19.1 against 11.3, 36608 x 5376
+//     at 24 54.4 against 37.5, 10624 x 11904 at 20 38.4 against 38.1).
+//   Not a single K block past 64 tokens, where its epilogue is the longer: 5248 x
+//     128 at 172 5.2 against 4.4, 2048 x 128 at 76 4.2 against 3.9.
 // Past 256 tokens there is no split, and 128 x 128 tiles that leave CUs idle take
 // 0.95 us for each 128 of K whatever their number: one round of smaller tiles is
 // the shorter.  4096 x 7168 at 320 / 512 tokens 45.6 / 47.5 against 53.8 / 54.9;
@@ -50,8 +54,8 @@ inline mid::Plan mid_plan(int M, int N, int K) {
   const mid::Plan p = mid::plan(M, N, K, kRound);
   const long long groups = p.ok ? (long long)p.tok_tiles * (N / (16 * mid::kTiles[p.tile].rt)) * p.splits : 0;
   const long long nk = (long long)N * K;
-  const bool small = K <= 3072 || nk <= 11500000 || (M <= 128 && nk <= 22100000);
-  return p.ok && (M <= 32 || (small && groups <= kRound)) ? p : mid::Plan{};
+  const bool small = M <= 32 || K <= 3072 || nk <= 11500000 || (M <= 128 && nk <= 22100000);
+  return p.ok && groups <= kRound && small && (K > 128 || M <= 64) ? p : mid::Plan{};
 }
 
 // fp32 partials of S splits.
@@ -65,8 +69,8 @@ struct Route {
 };
 
 // Each kernel asks for its own partials only: a workspace that holds the 128 x
-// 128 tiles' split but not the small tiles' (4224 x 3712 at 17 tokens: 2 against
-// 8 splits) still gets that split.  e4m3: the FP8 MFMA, which the small-tile
+// 128 tiles' split but not the small tiles' (128 x 1408 at 17 tokens: 4 against 8
+// splits) still gets that split.  e4m3: the FP8 MFMA, which the small-tile
 // kernel does not have.
 inline Route route(int M, int N, int K, bool e4m3, size_t ws_bytes) {
   Route r;

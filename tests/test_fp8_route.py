@@ -24,3 +24,20 @@ def test_each_kernel_asks_for_its_own_partials(tmp_path):
   }
   for (int M : {17, 100, 256}) for (int N : {128, 4096, 24576}) for (int K : {128, 1536, 7168, 16384})
     CHECK(f8::ue8m0_least_workspace(M, N, K) <= f8::ue8m0_workspace(M, N, K));""", "fp8_plan.hpp")
+
+
+def test_small_tiles_take_one_round(tmp_path):
+    """Past one round of work-groups, or a single K block past 64 tokens, the larger tiles are the faster."""
+    run_rules(tmp_path, r"""
+  for (int M = 17; M <= 256; ++M)
+    for (int N = 128; N <= 40960; N += 128)
+      for (int nkb : {1, 2, 7, 8, 16, 24, 56, 96, 128}) {
+        const mid::Plan p = f8::mid_plan(M, N, nkb * 128);
+        if (!p.ok) continue;
+        CHECK((long long)p.tok_tiles * (N / (16 * mid::kTiles[p.tile].rt)) * p.splits <= f8::kRound);
+        CHECK(nkb > 1 || M <= 64);
+      }
+  const int taken[][3] = {{24, 4096, 7168}, {32, 7168, 2048}, {64, 14720, 128}, {100, 4096, 512}, {256, 4096, 2048}};
+  for (auto& s : taken) CHECK(f8::mid_plan(s[0], s[1], s[2]).ok);
+  const int left[][3] = {{23, 34944, 1024}, {24, 36608, 5376}, {20, 10624, 11904}, {172, 5248, 128}, {100, 4096, 7168}};
+  for (auto& s : left) CHECK(!f8::mid_plan(s[0], s[1], s[2]).ok);""", "fp8_plan.hpp")

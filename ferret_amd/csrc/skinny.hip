@@ -408,11 +408,7 @@ int ferret_fp8_gemm_skinny(const void* a_, const float* sa, const void* b, const
   return launch_skinny<kFP8, kStore, 1>(a, (M + 15) / 16, st);
 }
 
-// Decode-sized FP8 MoE w13 (tile_m = 16).  Two tiles per unit from an average
-// of 6 rows per expert: at 9.4 rows an even routing, with hardly a second tile
-// anywhere, takes 1140 us either way, a Zipf(1.1) one 1238 against 1413 us
-// (6.3 rows: 1054 against 1130); below, an even routing loses the 0.8 % the
-// pairing costs (4 rows: 1086 against 1078 us).
+// Decode-sized FP8 MoE w13 (tile_m = 16).
 int ferret_moe_w13_fp8_skinny(const void* x, const float* sx, const void* w, const float* sw,
                               const int32_t* sorted_pair, const int32_t* tiles, const int32_t* ntiles,
                               int max_tiles, long long num_pairs, int topk, int E, int N, int K, void* out,
@@ -430,7 +426,7 @@ int ferret_moe_w13_fp8_skinny(const void* x, const float* sx, const void* w, con
   a.N = N;
   a.K = K;
   a.units_n = N / 32;
-  a.pair_tiles = num_pairs >= 6LL * E;
+  a.pair_tiles = moe::w13_pairs(num_pairs, E, N, K >> 7, cu_count());
   if (max_tiles <= 0) return FERRET_OK;
   const int rc = try_stream<kFP8, kSilu, 2, 3, 8>(a, 0, max_tiles, st);
   if (rc != 1) return rc;
@@ -439,8 +435,6 @@ int ferret_moe_w13_fp8_skinny(const void* x, const float* sx, const void* w, con
 
 // Decode-sized FP8 MoE w2 / down projection (tile_m = 16): the A row and the
 // output row of a sorted row are both its routed pair (topk = 1 indexing).
-// Two tiles per unit from an average of 10 rows per expert (15.6 rows: 652
-// against 870 us; 9.4 rows: 650 against 634 us).
 int ferret_moe_w2_fp8_skinny(const void* h, const float* sh, const void* w, const float* sw,
                              const int32_t* sorted_pair, const int32_t* tiles, const int32_t* ntiles,
                              int max_tiles, long long num_pairs, int E, int N, int K, void* out, hipStream_t st) {
@@ -465,7 +459,7 @@ int ferret_moe_w2_fp8_skinny(const void* h, const float* sh, const void* w, cons
 // 12 and 6 before, reached 4.2 TB/s of weights: 256 experts x 4 rows, N = 7168,
 // K = 1536 659 -> 425 us (6.5 TB/s); with 15 rows 1079 -> 552, K = 768 634 -> 350.
   a.units_n = N / 16;  // units of the per-unit fallback (RB = 1); try_stream derives its own
-  a.pair_tiles = num_pairs >= 10LL * E;
+  a.pair_tiles = moe::w2_pairs(num_pairs, E, N, K >> 7, cu_count());
   if (moe::w2_streams(K >> 7, w)) {
     int rc = try_stream<kFP8, kStore, 4, 3, 4>(a, 0, max_tiles, st);
     if (rc == 1) rc = try_half_stream<kFP8, kStore, 4, 3>(a, max_tiles, st);

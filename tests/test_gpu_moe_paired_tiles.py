@@ -13,13 +13,14 @@ import torch
 
 from oracle import gemm as G
 from tests.gpu_helpers import assert_gemm_close, bf16_out, codes8, f32
+from tests.test_linear_route import run_rules
 
 pytestmark = pytest.mark.gpu
 
 # one tile, exactly two, one row into the third, an odd and an even tile count; then a table past 512 rows
 # (two rounds of the table walk) whose runs cross its 64-row chunks
 EDGES = [1, 15, 16, 17, 0, 31, 32, 33, 48, 49, 64]
-MANY = [int(n) for n in np.random.default_rng(1).integers(1, 20, 600)]
+MANY = [int(n) for n in np.random.default_rng(1).integers(1, 31, 600)]
 
 
 @pytest.fixture(scope="module")
@@ -43,19 +44,20 @@ def _weights(E, N, K, padded):
     return w, sw
 
 
+# the sizes fill the CUs twice to sixteen times with units, as the rule of the paired kernel asks
 @pytest.mark.parametrize("which,rows,N,K", [
-    ("w13", EDGES, 512, 2048), ("w13", EDGES, 256, 4096), ("w13", EDGES, 768, 7168), ("w13", MANY, 256, 2048),
-    ("w2", EDGES, 384, 1024), ("w2", EDGES, 512, 2048), ("w2", EDGES, 128, 3584), ("w2", MANY, 128, 1024),
+    ("w13", EDGES, 6144, 2048), ("w13", EDGES, 3072, 4096), ("w13", EDGES, 3072, 7168), ("w13", MANY, 256, 2048),
+    ("w2", EDGES, 12032, 1024), ("w2", EDGES, 3072, 2048), ("w2", EDGES, 3200, 3584), ("w2", MANY, 512, 1024),
     # K / 128 of 12 (3 K-steps per wave), then 4, 6 and 14 (two work-groups of 2 waves per CU)
-    ("w2", EDGES, 256, 1536), ("w2", EDGES, 384, 512), ("w2", EDGES, 256, 768), ("w2", EDGES, 128, 1792),
+    ("w2", EDGES, 3072, 1536), ("w2", EDGES, 12032, 512), ("w2", EDGES, 3072, 768), ("w2", EDGES, 3200, 1792),
     ("w2", MANY, 128, 768)])
-def test_two_tiles_per_unit_equal_one(ops, which, rows, N, K):
+def test_two_tiles_per_unit_equal_one(ops, tmp_path, which, rows, N, K):
     from ferret_amd import workloads as W
     E, P = len(rows), sum(rows)
-    least = 6 if which == "w13" else 10
-    padded = min(1024, P // least + 1)
+    padded = min(1024, P // 6 + 1)
     print(f"[case] paired tiles {which} E={E} P={P} N={N} K={K}", flush=True)
-    assert P >= least * E and P < least * padded
+    run_rules(tmp_path, f"CHECK(moe::{which}_pairs({P}, {E}, {N}, {K // 128}, 256));"
+                        f"CHECK(!moe::{which}_pairs({P}, {padded}, {N}, {K // 128}, 256));", "moe_plan.hpp")
     ids = _ids(rows)
     x, sx = W.quant_act_1x128(W.randn((P, K), 11, "cuda"))
     w, sw = _weights(E, N, K, padded)

@@ -9,3 +9,17 @@ def test_w2_stream_kernel_takes_aligned_weights_only_where_another_kernel_is_lef
     const bool four = nkb == 8 || nkb == 16 || nkb == 28 || nkb == 32, more = nkb == 12 || nkb == 4 || nkb == 6 || nkb == 14;
     for (int off = 0; off <= 16; ++off) CHECK(moe::w2_streams(nkb, buf + off) == (four || (more && off % 16 == 0)));
   }""", "moe_plan.hpp")
+
+
+def test_two_tiles_per_unit_only_where_the_units_fill_the_cus(tmp_path):
+    """Few units, or hardly an expert with a second tile, keep one tile per unit."""
+    run_rules(tmp_path, r"""
+  // num_pairs, E, N, K / 128, taken
+  const int w13[][5] = {{5600, 256, 4096, 56, 1}, {1612, 256, 4096, 56, 1}, {1500, 256, 4096, 56, 0}, {260, 16, 512, 56, 0},
+    {600, 64, 512, 56, 0}, {480, 32, 1280, 56, 1}, {1904, 256, 512, 16, 0}, {194, 8, 256, 16, 0}, {416, 16, 256, 56, 0},
+    {6000, 256, 512, 16, 1}, {404, 32, 1280, 16, 0}};
+  for (auto& s : w13) CHECK(moe::w13_pairs(s[0], s[1], s[2], s[3], 256) == (s[4] != 0));
+  const int w2[][5] = {{4000, 256, 7168, 16, 1}, {2406, 256, 7168, 16, 0}, {1348, 128, 768, 16, 0}, {764, 64, 1536, 8, 0},
+    {362, 16, 1024, 8, 0}, {432, 16, 896, 28, 0}, {360, 32, 1152, 16, 0}, {6400, 256, 7168, 8, 1}, {4000, 256, 7168, 12, 1},
+    {4000, 256, 7168, 6, 1}, {4000, 256, 7168, 14, 1}};
+  for (auto& s : w2) CHECK(moe::w2_pairs(s[0], s[1], s[2], s[3], 256) == (s[4] != 0));""", "moe_plan.hpp")

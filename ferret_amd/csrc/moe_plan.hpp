@@ -13,11 +13,18 @@ inline bool w2_four_waves(int nkb) { return nkb == 8 || nkb == 16 || nkb == 28 |
 
 // Whether the stream kernel takes the w2 projection.  K / 128 = 12 (3 K-steps
 // per wave) and 4, 6 and 14 (two work-groups of 2 waves per CU) are the per-unit
-// kernel's otherwise; that one loads weights through registers, this one copies
-// them to LDS 16 bytes at a time, so tensors off that bound stay there.
-inline bool w2_streams(int nkb, const void* w) {
+// kernel's otherwise.  That one loads weights through registers, this one copies
+// them to LDS 16 bytes at a time, so tensors off that bound stay there; and its
+// units are 16 rows, not 64, so few tiles of few rows fill the CUs better.  The
+// line is in units (64 rows of a tile of the table) per CU, per-unit kernel /
+// this one (us) below and above it: K / 128 = 12, 1: 2 tiles of N = 2304 5.3 / 6.7,
+// above 1.14 times as fast (geometric mean of 47 shapes); 6 and 14, 3: 4 of 896,
+// K = 768 3.3 / 5.6, 8 of 640, K = 1792 5.0 / 6.9, above 1.14 and 1.19 times; 4, 8:
+// 10 of 512 3.3 / 4.7, 51 of 1408 9.0 / 9.9, above 1.03 times.
+inline bool w2_streams(int nkb, const void* w, long long units, int ncu) {
   if (w2_four_waves(nkb)) return true;
-  return (nkb == 12 || nkb == 4 || nkb == 6 || nkb == 14) && (reinterpret_cast<uintptr_t>(w) & 15) == 0;
+  const int least = nkb == 12 ? 1 : nkb == 6 || nkb == 14 ? 3 : nkb == 4 ? 8 : 0;
+  return least != 0 && units >= (long long)least * ncu && (reinterpret_cast<uintptr_t>(w) & 15) == 0;
 }
 
 // Whether a unit takes two 16-row tiles of an expert (stream kernel, TB = 2), from

@@ -460,7 +460,7 @@ int ferret_moe_w2_fp8_skinny(const void* h, const float* sh, const void* w, cons
 // K = 1536 659 -> 425 us (6.5 TB/s); with 15 rows 1079 -> 552, K = 768 634 -> 350.
   a.units_n = N / 16;  // units of the per-unit fallback (RB = 1); try_stream derives its own
   a.pair_tiles = moe::w2_pairs(num_pairs, E, N, K >> 7, cu_count());
-  if (moe::w2_streams(K >> 7, w)) {
+  if (moe::w2_streams(K >> 7, w, (long long)max_tiles * (N / 64), cu_count())) {
     int rc = try_stream<kFP8, kStore, 4, 3, 4>(a, 0, max_tiles, st);
     if (rc == 1) rc = try_half_stream<kFP8, kStore, 4, 3>(a, max_tiles, st);
     if (rc != 1) return rc;

@@ -73,11 +73,13 @@ def test_two_tiles_per_unit_equal_one(ops, tmp_path, which, rows, N, K):
         assert_gemm_close(bf16_out(got), ref, f"{which} N={N} K={K}")
 
 
-@pytest.mark.parametrize("K", [1536, 512, 768, 1792])
-def test_w2_weights_off_a_16_byte_bound(ops, K):
+@pytest.mark.parametrize("N,K", [(2048, 1536), (16384, 512), (6144, 768), (6144, 1792)])
+def test_w2_weights_off_a_16_byte_bound(ops, tmp_path, N, K):
     """K / 128 = 12, 4, 6 and 14: weights that start 8 bytes into a buffer keep the per-unit kernel."""
     from ferret_amd import workloads as W
-    E, N, P = 6, 256, 40
+    E, P = 6, 40
+    units = ops.moe_permute(torch.zeros((P, 1), dtype=torch.int32, device="cuda"), E, 16).max_tiles * (N // 64)
+    run_rules(tmp_path, f"CHECK(moe::w2_streams({K // 128}, (void*)64, {units}, 256));", "moe_plan.hpp")
     print(f"[case] w2 unaligned weights K={K}", flush=True)
     ids = torch.arange(P, device="cuda", dtype=torch.int32).remainder(E).view(-1, 1).contiguous()
     x, sx = W.quant_act_1x128(W.randn((P, K), 11, "cuda"))

@@ -2,12 +2,15 @@
 from tests.test_linear_route import run_rules
 
 
-def test_w2_stream_kernel_takes_aligned_weights_only_where_another_kernel_is_left(tmp_path):
+def test_w2_stream_kernel_takes_aligned_weights_and_many_units_where_another_kernel_is_left(tmp_path):
     run_rules(tmp_path, r"""
   alignas(64) static char buf[64];
   for (int nkb = 1; nkb <= 128; ++nkb) {
     const bool four = nkb == 8 || nkb == 16 || nkb == 28 || nkb == 32, more = nkb == 12 || nkb == 4 || nkb == 6 || nkb == 14;
-    for (int off = 0; off <= 16; ++off) CHECK(moe::w2_streams(nkb, buf + off) == (four || (more && off % 16 == 0)));
+    const int least = nkb == 12 ? 256 : nkb == 4 ? 2048 : 768;  // units
+    for (int off = 0; off <= 16; ++off)
+      for (int units : {1, least - 1, least, 100000})
+        CHECK(moe::w2_streams(nkb, buf + off, units, 256) == (four || (more && off % 16 == 0 && units >= least)));
   }""", "moe_plan.hpp")
 
 

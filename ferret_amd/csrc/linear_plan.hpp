@@ -74,6 +74,18 @@ inline bool tiled_aligned(const void* x, const void* w, const void* residual, co
 // fp32 partials of S splits.
 inline size_t partial_bytes(int S, int M, int N) { return S > 1 ? (size_t)S * M * N * sizeof(float) : 0; }
 
+// Workspace for tensors on the tiled kernel's bounds, and for any: where its plan
+// splits K less than the 16-token kernels (4432 x 16384 at 1036 tokens: 4 against 8),
+// those need the larger one for their split (unaligned x, 1647 us; 2513 without).
+inline size_t aligned_workspace(int M, int N, int K, int ncu) {
+  const bt::Plan tiled = tiled_plan(M, N, K, ncu);
+  return partial_bytes(tiled.ok ? tiled.splits : stream_splits(M, N, K, ncu), M, N);
+}
+inline size_t workspace(int M, int N, int K, int ncu) {
+  const size_t tiled = aligned_workspace(M, N, K, ncu), units = partial_bytes(stream_splits(M, N, K, ncu), M, N);
+  return tiled > units ? tiled : units;
+}
+
 // What a call runs: the LDS-tiled kernel by `tiled` where that is ok, else the
 // 16-token kernels with K split by `splits`.
 struct Route {

@@ -146,6 +146,12 @@ PyObject* wrap(const at::Tensor& t) { return THPVariable_Wrap(t); }
   }                                                                                            \
   PyObject* name##_body(PyObject* const* a)
 
+// The bounds of ferret_workspace_bytes(6, ...).
+bool on_bounds(const void* x, const void* w, const void* residual, const void* y) {
+  const auto bits = [](const void* p) { return reinterpret_cast<uintptr_t>(p); };
+  return ((bits(x) | bits(w)) & 15) == 0 && ((bits(residual) | bits(y)) & 7) == 0;
+}
+
 // x, w, residual, out, workspace
 NATIVE(linear_bf16, 5) {
   Call c;
@@ -158,12 +164,13 @@ NATIVE(linear_bf16, 5) {
   if (!c.ok() || (r != nullptr && (r->size(0) != M || r->size(1) != N))) Py_RETURN_NONE;
   const at::Tensor y = c.out(a[3], {M, N}, kBf16);
   if (!c.ok()) Py_RETURN_NONE;
-  const size_t need = K % 128 == 0 && N % 16 == 0 ? ferret_workspace_bytes(0, M, N, K, 0) : 0;
+  void *xp = ptr(x), *wp = ptr(w), *rp = r ? ptr(r) : nullptr, *yp = ptr(y);
+  const size_t need = ferret_workspace_bytes(on_bounds(xp, wp, rp, yp) ? 6 : 0, M, N, K, 0);
   const at::Tensor ws = c.workspace(a[4], need);
   if (!c.ok()) Py_RETURN_NONE;
   void* st = stream();
-  if (!run([&] { return ferret_linear_bf16(ptr(x), ptr(w), r ? ptr(r) : nullptr, ptr(y), M, N, K, ptr(ws), need, st); }))
-    Py_RETURN_NONE;
+  const size_t have = ws.defined() ? ws.nbytes() : 0;
+  if (!run([&] { return ferret_linear_bf16(xp, wp, rp, yp, M, N, K, ptr(ws), have, st); })) Py_RETURN_NONE;
   return wrap(y);
 }
 

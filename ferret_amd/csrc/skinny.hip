@@ -242,12 +242,10 @@ static int launch_bf16_tiled_serial(const bt::Plan& plan, const SkinnyArgs& a, h
 
 using namespace ferret;
 
-static size_t linear_workspace(const bt::Plan& tiled, int M, int N, int K) {
-  return lin::partial_bytes(tiled.ok ? tiled.splits : lin::stream_splits(M, N, K, cu_count()), M, N);
-}
+size_t ferret_linear_bf16_workspace(int M, int N, int K) { return lin::workspace(M, N, K, cu_count()); }
 
-size_t ferret_linear_bf16_workspace(int M, int N, int K) {
-  return linear_workspace(lin::tiled_plan(M, N, K, cu_count()), M, N, K);
+size_t ferret_linear_bf16_aligned_workspace(int M, int N, int K) {
+  return lin::aligned_workspace(M, N, K, cu_count());
 }
 
 extern "C" int ferret_linear_bf16(const void* x, const void* w, const void* residual, void* y, int M,
@@ -341,7 +339,7 @@ extern "C" int ferret_linear_bf16_noalloc(const void* x, const void* w, const vo
   const int splits = lin::stream_splits(M, N, K, cu_count());
   FERRET_REQUIRE(splits <= 1 || (size_t)splits * M * N * sizeof(float) <= kNoAllocScratchBytes, FERRET_ERR_WORKSPACE);
   const bt::Plan tiled = lin::tiled_plan(M, N, K, cu_count());
-  const size_t need = linear_workspace(tiled, M, N, K);
+  const size_t need = lin::partial_bytes(tiled.splits, M, N);
   SkinnyArgs a{};
   a.w = static_cast<const uint8_t*>(w);
   a.x = static_cast<const uint8_t*>(x);

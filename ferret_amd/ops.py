@@ -90,12 +90,14 @@ def linear_bf16(x: torch.Tensor, w: torch.Tensor, residual: torch.Tensor | None 
     rp = 0
     if residual is not None:
         rp = _out(residual, "residual", (M, N), torch.bfloat16, x.device)
-    need = linear_workspace_bytes(M, N, K) if K % 128 == 0 and N % 16 == 0 else 0
+    on_bounds = (x.data_ptr() | w.data_ptr()) % 16 == 0 and (rp | out.data_ptr()) % 8 == 0
+    need = int(_lib.load().ferret_workspace_bytes(6 if on_bounds else 0, M, N, K, 0))
     if need and (workspace is None or workspace.numel() * workspace.element_size() < need):
         workspace = torch.empty(need, dtype=torch.uint8, device=x.device)
     rc = _lib.load().ferret_linear_bf16(_dev(x, "x", torch.bfloat16, 2), _dev(w, "w", torch.bfloat16, 2), rp,
                                         _dev(out, "out", torch.bfloat16, 2), M, N, K,
-                                        _dev(workspace, "workspace") if need else None, need, _stream())
+                                        _dev(workspace, "workspace") if need else None,
+                                        workspace.numel() * workspace.element_size() if need else 0, _stream())
     _lib.check("ferret_linear_bf16", rc)
     return out
 

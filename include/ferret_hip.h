@@ -298,7 +298,9 @@ int ferret_moe_w2_fp8_ex(const void* h, const float* sh, const void* w, const fl
 /* Workspace bytes an op can use (0 = none). op: 0 linear_bf16 (split-K partials),
  * 1 fp8_gemm_blockscale (split-K partials for 16 < M <= 256), 2 moe_w13_fp8,
  * 3 moe_w13_w4a16, 4 moe_permute (M = number of routed pairs P, E experts),
- * 5 fp8_gemm_ue8m0 (decoded scales + split-K partials; required). */
+ * 5 fp8_gemm_ue8m0 (decoded scales + split-K partials; required), 6 linear_bf16
+ * where x and w start on 16-byte and residual and y on 8-byte bounds (less than
+ * 0 where only other tensors need it). */
 size_t ferret_workspace_bytes(int op, int M, int N, int K, int E);
 
 #ifdef __cplusplus

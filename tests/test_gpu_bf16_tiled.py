@@ -157,3 +157,15 @@ def test_allocation_free_calls_without_a_16_token_split_may_overlap(hip):
     torch.cuda.synchronize()
     for out, y in zip(outs, want):
         assert all(torch.equal(o.view(torch.int16), y.view(torch.int16)) for o in out)
+
+
+@pytest.mark.parametrize("M,N,K,off", [(512, 4096, 6144, 4), (64, 8192, 6144, 4), (64, 8192, 6144, 0)])
+def test_default_workspace_serves_both_kernels(ops, hip, M, N, K, off):
+    """Shapes that the tiled plan splits less than the 16-token kernels, through the entry point that allocates."""
+    on, any_ = (int(hip.ferret_workspace_bytes(op, M, N, K, 0)) for op in (6, 0))
+    print(f"[case] bf16 default workspace M={M} N={N} K={K} off={off} bytes {on} {any_}", flush=True)
+    assert on < any_ == 3 * M * N * 4
+    x, w, r = _inputs(M, N, K, True)
+    y = ops.linear_bf16(_at(x, off), w, r)
+    torch.cuda.synchronize()
+    assert_gemm_close(bf16_out(y), G.linear_bf16(bits16(x), bits16(w), bits16(r)), "default workspace")

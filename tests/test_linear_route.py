@@ -70,3 +70,19 @@ def test_each_kernel_asks_for_its_own_partials(tmp_path):
   }
   const int unsplit[3] = {64, 24576, 4096};  // needs no workspace and looks at none
   CHECK(route(unsplit, 0, 0, false).tiled.ok && lin::route(64, 24576, 4096, 256, b[0], b[1], b[2], b[3], b[4] + 1, 8).tiled.ok);""")
+
+
+def test_reported_workspace_serves_tensors_on_and_off_the_bounds(tmp_path):
+    """Where the tiled plan splits less than the 16-token kernels, unaligned tensors find their split all the same."""
+    run_rules(tmp_path, r"""
+  alignas(64) static char b[5][64];
+  // M, N, K, splits of the tiled plan and of the 16-token kernels
+  const int shapes[][5] = {{512, 4096, 12288, 2, 3}, {2048, 8192, 6144, 1, 3}, {1036, 4432, 16384, 4, 8}, {48, 4096, 12288, 4, 3}};
+  for (auto& s : shapes) {
+    const int M = s[0], N = s[1], K = s[2];
+    const size_t any = lin::workspace(M, N, K, 256), on = lin::aligned_workspace(M, N, K, 256);
+    CHECK(lin::stream_splits(M, N, K, 256) == s[4] && on == lin::partial_bytes(s[3], M, N));
+    CHECK(any == lin::partial_bytes(s[3] > s[4] ? s[3] : s[4], M, N));
+    CHECK(lin::route(M, N, K, 256, b[0], b[1], b[2], b[3], b[4], on).tiled.splits == s[3]);
+    CHECK(lin::route(M, N, K, 256, b[0] + 8, b[1], b[2], b[3], b[4], any).splits == s[4]);
+  }""")

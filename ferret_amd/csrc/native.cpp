@@ -10,8 +10,9 @@
 // its result, or None whenever anything is not the plain case: an argument that
 // is no exact torch.Tensor (or Parameter), not a contiguous GPU tensor of the
 // expected type and shape, wrapped by a transform, under a dispatch or function
-// mode, or a non-zero return code.  The caller (ops.py) then takes its Python
-// path, which names the error or handles the case.
+// mode, or a rejected argument (a negative return code).  The caller (ops.py) then
+// takes its Python path, which names the error or handles the case.  A HIP error
+// (a positive code) is raised at once (native_run.hpp).
 #include <Python.h>
 #include <ATen/ATen.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
@@ -23,8 +24,12 @@
 #include <climits>
 
 #include "../../include/ferret_hip.h"
+#include "native_run.hpp"
 
 namespace {
+
+using ferret::native::declined;
+using ferret::native::run;
 
 constexpr auto kBf16 = at::kBFloat16;
 constexpr auto kF32 = at::kFloat;
@@ -114,16 +119,6 @@ T* ptr_as(const at::Tensor* t) { return static_cast<T*>(t->data_ptr()); }
 
 void* stream() { return c10::hip::getCurrentHIPStream().stream(); }
 
-// The C-ABI call without the interpreter lock (as ctypes makes it).
-template <typename F>
-bool run(F&& f) {
-  int rc;
-  Py_BEGIN_ALLOW_THREADS
-  rc = f();
-  Py_END_ALLOW_THREADS
-  return rc == FERRET_OK;
-}
-
 bool as_int(PyObject* o, int* v) {
   const long x = PyLong_CheckExact(o) ? PyLong_AsLong(o) : -1;
   if (PyErr_Occurred() != nullptr) PyErr_Clear();
@@ -170,7 +165,8 @@ NATIVE(linear_bf16, 5) {
   if (!c.ok()) Py_RETURN_NONE;
   void* st = stream();
   const size_t have = ws.defined() ? ws.nbytes() : 0;
-  if (!run([&] { return ferret_linear_bf16(xp, wp, rp, yp, M, N, K, ptr(ws), have, st); })) Py_RETURN_NONE;
+  if (!run("ferret_linear_bf16", [&] { return ferret_linear_bf16(xp, wp, rp, yp, M, N, K, ptr(ws), have, st); }))
+    return declined();
   return wrap(y);
 }
 
@@ -192,11 +188,11 @@ NATIVE(fp8_gemm_blockscale, 7) {
   const at::Tensor ws = c.workspace(a[5], need);
   if (!c.ok()) Py_RETURN_NONE;
   void* st = stream();
-  if (!run([&] {
+  if (!run("ferret_fp8_gemm_blockscale", [&] {
         return ferret_fp8_gemm_blockscale_ex(ptr(x), ptr_as<float>(sx), ptr(w), ptr_as<float>(sw), ptr(y), M, N, K,
                                              ptr(ws), need, flags, st);
       }))
-    Py_RETURN_NONE;
+    return declined();
   return wrap(y);
 }
 
@@ -217,11 +213,11 @@ NATIVE(fp8_gemm_ue8m0, 6) {
   const at::Tensor ws = c.workspace(a[5], need);
   if (!c.ok()) Py_RETURN_NONE;
   void* st = stream();
-  if (!run([&] {
+  if (!run("ferret_fp8_gemm_ue8m0", [&] {
         return ferret_fp8_gemm_ue8m0(ptr(x), ptr_as<uint32_t>(sx), ptr(w), ptr_as<uint32_t>(sw), ptr(y), M, N, K,
                                      ptr(ws), ws.nbytes(), st);
       }))
-    Py_RETURN_NONE;
+    return declined();
   return wrap(y);
 }
 
@@ -238,10 +234,10 @@ NATIVE(moe_route_topk, 3) {
   const at::Tensor ids = c.fresh({T, topk}, kI32);
   const at::Tensor w = with_weights ? c.fresh({T, topk}, kF32) : at::Tensor();
   void* st = stream();
-  if (!run([&] {
+  if (!run("ferret_moe_route_topk", [&] {
         return ferret_moe_route_topk(ptr_as<float>(x), T, E, topk, ptr_as<int32_t>(ids), ptr_as<float>(w), st);
       }))
-    Py_RETURN_NONE;
+    return declined();
   PyObject* pw = Py_None;
   if (with_weights) pw = wrap(w);
   else Py_INCREF(pw);
@@ -268,12 +264,12 @@ NATIVE(moe_permute, 4) {
                    sorted_pair = c.fresh({std::max<int64_t>(P, 1)}, kI32), tiles = c.fresh({max_tiles, 3}, kI32),
                    ntiles = c.fresh({1}, kI32);
   void* st = stream();
-  if (!run([&] {
+  if (!run("ferret_moe_permute", [&] {
         return ferret_moe_permute(ptr_as<int32_t>(ids), T, topk, E, tile_m, ptr_as<int32_t>(counts),
                                   ptr_as<int32_t>(offsets), ptr_as<int32_t>(sorted_pair), ptr_as<int32_t>(tiles),
                                   max_tiles, ptr_as<int32_t>(ntiles), ptr(ws), need, st);
       }))
-    Py_RETURN_NONE;
+    return declined();
   return Py_BuildValue("(NNNNNiiii)", wrap(counts), wrap(offsets), wrap(sorted_pair), wrap(tiles), wrap(ntiles),
                        tile_m, max_tiles, topk, T);
 }
@@ -308,13 +304,13 @@ NATIVE(moe_w13_fp8, 14) {
   const at::Tensor y = c.out(a[12], {P, N / 2}, kBf16);
   if (!c.ok()) Py_RETURN_NONE;
   void* st = stream();
-  if (!run([&] {
+  if (!run("ferret_moe_w13_fp8", [&] {
         return ferret_moe_w13_fp8_ex(ptr(x), ptr_as<float>(sx), ptr(w), ptr_as<float>(sw),
                                      ptr_as<int32_t>(rt.sorted_pair), ptr_as<int32_t>(rt.tiles),
                                      ptr_as<int32_t>(rt.ntiles), rt.max_tiles, rt.tile_m, T, rt.topk, E, N, K, ptr(y),
                                      flags, st);
       }))
-    Py_RETURN_NONE;
+    return declined();
   return wrap(y);
 }
 
@@ -334,12 +330,12 @@ NATIVE(moe_w2_fp8, 14) {
   const at::Tensor y = c.out(a[12], {P, N}, kBf16);
   if (!c.ok()) Py_RETURN_NONE;
   void* st = stream();
-  if (!run([&] {
+  if (!run("ferret_moe_w2_fp8", [&] {
         return ferret_moe_w2_fp8_ex(ptr(h), ptr_as<float>(sh), ptr(w), ptr_as<float>(sw),
                                     ptr_as<int32_t>(rt.sorted_pair), ptr_as<int32_t>(rt.tiles),
                                     ptr_as<int32_t>(rt.ntiles), rt.max_tiles, rt.tile_m, P, E, N, K, ptr(y), flags, st);
       }))
-    Py_RETURN_NONE;
+    return declined();
   return wrap(y);
 }
 
@@ -361,7 +357,7 @@ NATIVE(moe_w13_w4a16, 12) {
   const at::Tensor y = c.out(a[11], {P, N / 2}, kBf16);
   if (!c.ok()) Py_RETURN_NONE;
   void* st = stream();
-  if (!run([&] {
+  if (!run(tiled ? "ferret_moe_w13_w4a16_tiled" : "ferret_moe_w13_w4a16", [&] {
         if (tiled)
           return ferret_moe_w13_w4a16_tiled(ptr(x), ptr(wq), ptr(ws), ptr_as<int32_t>(rt.sorted_pair),
                                             ptr_as<int32_t>(rt.tiles), ptr_as<int32_t>(rt.ntiles), rt.max_tiles,
@@ -370,7 +366,7 @@ NATIVE(moe_w13_w4a16, 12) {
                                     ptr_as<int32_t>(rt.tiles), ptr_as<int32_t>(rt.ntiles), rt.max_tiles, rt.tile_m, T,
                                     rt.topk, E, N, K, ptr(y), st);
       }))
-    Py_RETURN_NONE;
+    return declined();
   return wrap(y);
 }
 
@@ -384,7 +380,9 @@ NATIVE(quant_act_e4m3, 3) {
   const at::Tensor s = c.out(a[2], {M, K / 128}, kF32);
   if (!c.ok()) Py_RETURN_NONE;
   void* st = stream();
-  if (!run([&] { return ferret_quant_act_e4m3(ptr(x), ptr(q), ptr_as<float>(s), M, K, st); })) Py_RETURN_NONE;
+  if (!run("ferret_quant_act_e4m3",
+           [&] { return ferret_quant_act_e4m3(ptr(x), ptr(q), ptr_as<float>(s), M, K, st); }))
+    return declined();
   return Py_BuildValue("(NN)", wrap(q), wrap(s));
 }
 
@@ -399,7 +397,9 @@ NATIVE(moe_combine, 3) {
   const at::Tensor y = c.out(a[2], {T, N}, kBf16);
   if (!c.ok()) Py_RETURN_NONE;
   void* st = stream();
-  if (!run([&] { return ferret_moe_combine(ptr(o), ptr_as<float>(w), T, topk, N, ptr(y), st); })) Py_RETURN_NONE;
+  if (!run("ferret_moe_combine",
+           [&] { return ferret_moe_combine(ptr(o), ptr_as<float>(w), T, topk, N, ptr(y), st); }))
+    return declined();
   return wrap(y);
 }
 

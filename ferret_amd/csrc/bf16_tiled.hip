@@ -19,9 +19,9 @@
 // plan, G at a time, and sums them itself, in the order and from the K rotation
 // of the plan's own tiles: their results bit for bit with no partials in memory.
 // For the allocation-free entry where the 16-token kernels need no split, so that
-// calls there share no memory.  Over 1200 such shapes of 1 .. 128 tokens 1.44
-// times as fast as those kernels (geometric mean; 75 of them slower, by 3 - 28 %),
-// the split form 1.70 times.
+// calls there share no memory.  Over 1468 such shapes of 1 .. 128 tokens 1.43
+// times as fast as those kernels (geometric mean; 43 of them more than 4 % slower,
+// by up to 33 %), the split form about 1.7 times.
 //
 // Measured, start to now (the 16-token stream kernel once per 16 tokens):
 // 4096 x 12288 + residual at 48 tokens 53.4 -> 23 us, 24576 x 4096 at 64 tokens
@@ -268,13 +268,19 @@ int ferret_bf16_tiled_serial(int tile, ferret::bt::Args p, hipStream_t st) {
   p.rot_rows = 16 * kTiles[tile].rt;
   // Few rows leave CUs idle where a work-group takes all tokens: below 2560 of
   // them it takes 16 (geometric means against the 16-token kernels: 1.28 - 1.75
-  // there against 0.55 - 1.2; from 2560 rows on 1.0 - 1.7 against 1.3 - 3).
-  if (p.M <= 16 && tile < 6) return launch_serial<1, 128, 4, 1, 4, 4>(p, st);
-  if (p.M <= 16 || p.N < 2560) {
+  // there against 0.55 - 1.2; from 2560 rows on 1.0 - 1.7 against 1.3 - 3).  As
+  // many splits at a time as the plan has, or a quarter to all of the waves idle:
+  // 10304 x 3072 at 2 tokens (3 splits) 26.3 us with 8 at a time, 13.8 with 4; 7664
+  // x 1536 at 9 (2 splits) 8.9 with 4, 6.4 with 2.  Plans of 64 K a stage pick their
+  // 128-token tile for few tokens too: up to 32 it takes 16 (6368 x 7168 at 25 53.1
+  // us with 128).
+  if (p.M <= 16 && tile < 6)
+    return p.splits <= 2 ? launch_serial<1, 128, 4, 1, 4, 2>(p, st) : launch_serial<1, 128, 4, 1, 4, 4>(p, st);
+  if (p.M <= 16 || p.N < 2560 || (tile == 12 && p.M <= 32)) {
     if (tile < 6) return launch_serial<1, 128, 2, 1, 4, 4>(p, st);
     if (tile < 10) return launch_serial<1, 128, 2, 1, 2, 4>(p, st);
     if (tile < 12) return launch_serial<1, 128, 2, 1, 1, 4>(p, st);
-    return launch_serial<1, 64, 2, 1, 1, 8>(p, st);
+    return p.splits <= 4 ? launch_serial<1, 64, 4, 1, 1, 4>(p, st) : launch_serial<1, 64, 2, 1, 1, 8>(p, st);
   }
   switch (tile) {
     case 0: case 1: return FERRET_ERR_SHAPE;  // 16 tokens: above

@@ -127,7 +127,7 @@ def _workspace_bits(hip, x, w, r, M, N, K):
     (33, 1440, 2432, True), (33, 3280, 1664, False), (50, 1584, 1664, True), (50, 4224, 1280, False),
     (70, 1824, 1152, True), (100, 592, 2560, False), (70, 3360, 1280, True), (100, 1648, 1280, False),
     (100, 2144, 1408, True), (97, 2720, 1152, True), (200, 1008, 2816, False), (5, 6368, 1664, True),
-    (200, 2704, 1792, False),
+    (200, 2704, 1792, False), (6, 7616, 1664, True), (2, 10304, 3072, False), (25, 6368, 7168, True), (1, 6352, 1664, True),
     (48, 4096, 12288, True), (64, 4096, 12288, True), (80, 4096, 12288, False)])
 def test_allocation_free_entry_gives_the_same_bits_on_every_tile(hip, M, N, K, res):
     print(f"[case] bf16 tiled noalloc M={M} N={N} K={K} res={res}", flush=True)

@@ -15,6 +15,19 @@ inline void raise_code(const char* entry, int rc) {
   Py_XDECREF(lib);
 }
 
+// The interpreter lock given up for a scope.  Taken back also where a C++
+// exception leaves it: the function's handler sets a Python error, which needs it.
+class Unlocked {
+ public:
+  Unlocked() : state_(PyEval_SaveThread()) {}
+  ~Unlocked() { PyEval_RestoreThread(state_); }
+  Unlocked(const Unlocked&) = delete;
+  Unlocked& operator=(const Unlocked&) = delete;
+
+ private:
+  PyThreadState* state_;
+};
+
 // f() is the C call of `entry`, made without the interpreter lock (as ctypes
 // makes it).  True where it returned 0.  A negative code was returned before
 // anything was launched: the Python path makes the call again and names the
@@ -24,9 +37,10 @@ inline void raise_code(const char* entry, int rc) {
 template <typename F>
 bool run(const char* entry, F&& f) {
   int rc;
-  Py_BEGIN_ALLOW_THREADS
-  rc = f();
-  Py_END_ALLOW_THREADS
+  {
+    const Unlocked unlocked;
+    rc = f();
+  }
   if (rc > 0) raise_code(entry, rc);
   return rc == 0;
 }

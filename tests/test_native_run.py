@@ -14,6 +14,7 @@ CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))),
 
 MODULE = r"""
 #include "native_run.hpp"
+#include <stdexcept>
 using namespace ferret::native;
 static int calls = 0;
 static PyObject* call(PyObject*, PyObject* code) {
@@ -21,8 +22,18 @@ static PyObject* call(PyObject*, PyObject* code) {
   if (!run("ferret_entry", [&] { ++calls; return rc; })) return declined();
   return PyUnicode_FromString("done");
 }
+static PyObject* fail(PyObject*, PyObject*) {
+  try {
+    run("ferret_entry", []() -> int { throw std::runtime_error("no storage"); });
+  } catch (const std::exception& e) {  // as the functions of native.cpp do
+    PyErr_SetString(PyExc_RuntimeError, e.what());
+    return nullptr;
+  }
+  Py_RETURN_NONE;
+}
 static PyObject* count(PyObject*, PyObject*) { return PyLong_FromLong(calls); }
-static PyMethodDef kMethods[] = {{"call", call, METH_O, nullptr}, {"count", count, METH_NOARGS, nullptr},
+static PyMethodDef kMethods[] = {{"call", call, METH_O, nullptr}, {"fail", fail, METH_NOARGS, nullptr},
+                                 {"count", count, METH_NOARGS, nullptr},
                                  {nullptr, nullptr, 0, nullptr}};
 static PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "run_probe", "", -1, kMethods, nullptr, nullptr, nullptr, nullptr};
 PyMODINIT_FUNC PyInit_run_probe(void) { return PyModule_Create(&kModule); }
@@ -60,3 +71,9 @@ def test_hip_errors_are_raised_and_rejected_arguments_left_to_python(probe, monk
         probe.call(719)
     assert e.value.code == 719
     assert probe.count() == before + 3      # each code came from one call
+
+
+def test_a_cpp_exception_leaves_the_interpreter_lock_held(probe):
+    """A pointer taken inside the call can throw (a tensor without storage, a copy-on-write one out of memory)."""
+    with pytest.raises(RuntimeError, match="no storage"):
+        probe.fail()

@@ -118,15 +118,29 @@ def build(verbose: bool = False) -> str:
     return LIB
 
 
-def build_native() -> str:
-    """Compile csrc/native.cpp (host code only) against torch and the library."""
+def build_native() -> str | None:
+    """Compile csrc/native.cpp (host code only) against torch and the library.
+
+    Where torch or g++ is absent it is left out (None): the library, and a
+    program on its C ABI, need neither, and ferret_amd.ops works without it.  An
+    earlier build is removed then, as it belongs to another library.
+    """
     import sysconfig
 
-    import torch
+    gxx = shutil.which("g++")
+    try:
+        import torch
+    except ImportError:
+        torch = None
+    if torch is None or gxx is None:
+        if os.path.exists(NATIVE):
+            os.remove(NATIVE)
+        print(f"{'torch' if torch is None else 'g++'} not found: {os.path.basename(NATIVE)} left out", file=sys.stderr)
+        return None
 
     troot = os.path.dirname(torch.__file__)
     tmp = NATIVE + ".tmp"
-    cmd = [shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall",
+    cmd = [gxx, "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall",
            "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", f"-I{troot}/include", f"-I{troot}/include/torch/csrc/api/include",
            f"-I{os.path.join(os.path.dirname(os.path.dirname(hipcc())), 'include')}", "-I/opt/rocm/include",
            f"-I{sysconfig.get_paths()['include']}",

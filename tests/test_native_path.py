@@ -7,6 +7,8 @@ bits of the Python path, and the errors stay that path's own.
 from __future__ import annotations
 
 import os
+import shutil
+import sys
 
 import pytest
 import torch
@@ -34,6 +36,32 @@ def test_modes_are_left_to_python(native):
     from torch._subclasses.fake_tensor import FakeTensorMode
     with FakeTensorMode():
         assert native.quant_act_e4m3(torch.zeros(2, 128, dtype=torch.bfloat16, device="cuda"), None, None) is None
+
+
+def test_without_the_module_operators_take_the_python_path(native, monkeypatch, tmp_path):
+    monkeypatch.setattr(lib, "_NATIVE", None)
+    monkeypatch.setattr(lib, "NATIVE_PATH", str(tmp_path / "_native.so"))
+    with pytest.warns(RuntimeWarning, match="_native.so is missing"):
+        nat = lib.native()
+    assert nat.linear_bf16(None, None, None, None, None) is None
+    assert lib.native() is nat      # warned of once
+    from ferret_amd import ops
+    with pytest.raises(ValueError, match="GPU tensor"):
+        ops.linear_bf16(torch.zeros(2, 128, dtype=torch.bfloat16), torch.zeros(16, 128, dtype=torch.bfloat16))
+
+
+@pytest.mark.parametrize("absent", ["torch", "g++"])
+def test_the_library_builds_without_what_only_the_module_needs(monkeypatch, tmp_path, absent):
+    from ferret_amd import build
+    stale = tmp_path / "_native.so"
+    stale.write_bytes(b"")
+    monkeypatch.setattr(build, "NATIVE", str(stale))
+    if absent == "torch":
+        monkeypatch.setitem(sys.modules, "torch", None)
+    else:
+        which = shutil.which
+        monkeypatch.setattr(build.shutil, "which", lambda name: None if name == "g++" else which(name))
+    assert build.build_native() is None and not stale.exists()
 
 
 def _moe(ops):

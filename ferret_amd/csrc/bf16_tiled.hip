@@ -243,7 +243,7 @@ static int launch_serial(Args p, hipStream_t st) {
 
 int ferret_bf16_tiled(int tile, const ferret::bt::Args& p, hipStream_t st) {
   using namespace ferret::bt;
-  static_assert(kNumTiles == 13, "one case per tile");
+  static_assert(kNumTiles == 12, "one case per tile");
   switch (tile) {
     case 0: return launch<0, 2, 1, 4>(p, st);
     case 1: return launch<1, 2, 1, 4>(p, st);
@@ -257,14 +257,13 @@ int ferret_bf16_tiled(int tile, const ferret::bt::Args& p, hipStream_t st) {
     case 9: return launch<9, 2, 2, 2>(p, st);
     case 10: return launch<10, 2, 4, 1>(p, st);
     case 11: return launch<11, 2, 4, 1>(p, st);
-    case 12: return launch<12, 2, 4, 1>(p, st);
   }
   return FERRET_ERR_SHAPE;
 }
 
 int ferret_bf16_tiled_serial(int tile, ferret::bt::Args p, hipStream_t st) {
   using namespace ferret::bt;
-  static_assert(kNumTiles == 13, "one case per tile");
+  static_assert(kNumTiles == 12, "one case per tile");
   p.rot_rows = 16 * kTiles[tile].rt;
   // Few rows leave CUs idle where a work-group takes all tokens: below 2560 of
   // them it takes 16 (geometric means against the 16-token kernels: 1.28 - 1.75
@@ -276,10 +275,10 @@ int ferret_bf16_tiled_serial(int tile, ferret::bt::Args p, hipStream_t st) {
   // us with 128).
   if (p.M <= 16 && tile < 6)
     return p.splits <= 2 ? launch_serial<1, 128, 4, 1, 4, 2>(p, st) : launch_serial<1, 128, 4, 1, 4, 4>(p, st);
-  if (p.M <= 16 || p.N < 2560 || (tile == 12 && p.M <= 32)) {
+  if (p.M <= 16 || p.N < 2560 || (tile == 11 && p.M <= 32)) {
     if (tile < 6) return launch_serial<1, 128, 2, 1, 4, 4>(p, st);
     if (tile < 10) return launch_serial<1, 128, 2, 1, 2, 4>(p, st);
-    if (tile < 12) return launch_serial<1, 128, 2, 1, 1, 4>(p, st);
+    if (tile < 11) return launch_serial<1, 128, 2, 1, 1, 4>(p, st);
     return p.splits <= 4 ? launch_serial<1, 64, 4, 1, 1, 4>(p, st) : launch_serial<1, 64, 2, 1, 1, 8>(p, st);
   }
   switch (tile) {
@@ -288,8 +287,8 @@ int ferret_bf16_tiled_serial(int tile, ferret::bt::Args p, hipStream_t st) {
     case 4: case 5: return launch_serial<3, 128, 5, 1, 4, 1>(p, st);
     case 6: case 7: return launch_serial<4, 128, 4, 2, 2, 1>(p, st);
     case 8: case 9: return launch_serial<6, 128, 4, 2, 2, 1>(p, st);
-    case 10: case 11: return launch_serial<8, 128, 4, 4, 1, 1>(p, st);
-    case 12: return launch_serial<8, 64, 4, 4, 1, 1>(p, st);
+    case 10: return launch_serial<8, 128, 4, 4, 1, 1>(p, st);
+    case 11: return launch_serial<8, 64, 4, 4, 1, 1>(p, st);
   }
   return FERRET_ERR_SHAPE;
 }

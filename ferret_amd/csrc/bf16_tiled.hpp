@@ -29,7 +29,7 @@ struct Tile {
 };
 constexpr Tile kTiles[] = {
     {4, 1, 128, 4}, {6, 1, 128, 5}, {4, 2, 128, 5}, {6, 2, 128, 5}, {4, 3, 128, 5}, {6, 3, 128, 4},
-    {4, 4, 128, 4}, {6, 4, 128, 4}, {4, 6, 128, 4}, {6, 6, 128, 3}, {4, 8, 128, 3}, {6, 8, 128, 2}, {8, 8, 64, 4}};
+    {4, 4, 128, 4}, {6, 4, 128, 4}, {4, 6, 128, 4}, {6, 6, 128, 3}, {4, 8, 128, 3}, {8, 8, 64, 4}};
 constexpr int kNumTiles = sizeof(kTiles) / sizeof(kTiles[0]);
 
 struct Plan {
@@ -45,9 +45,9 @@ constexpr int kMaxTokenSplits = 8192;
 
 // The tile and K split with the least estimated time.  A stage takes what its
 // weights take at 25 B/ns per CU (6.4 TB/s from HBM over 256 CUs) or, where
-// larger, what all its bytes take through a CU's loads (46 B/ns, 36 with one
-// stage in flight); a round of work-groups adds 1.5 us of pipeline fill and
-// epilogue, a split the reduce launch and the fp32 partials' way out and back.
+// larger, what all its bytes take through a CU's loads (46 B/ns); a round of
+// work-groups adds 1.5 us of pipeline fill and epilogue, a split the reduce launch
+// and the fp32 partials' way out and back.
 // Measured against the model: 4096 x 12288 at 64 tokens 24.2 / 25.3 us, 24576 x
 // 4096 at 64 tokens 34.2 / 35.9 us, at 128 tokens 51.6 / 52.1 us.
 inline Plan plan(int M, int N, int K, int ncu) {
@@ -61,7 +61,7 @@ inline Plan plan(int M, int N, int K, int ncu) {
     if (tok_tiles > 1 && t.tt < 6) continue;
     const long long tiles = tok_tiles * ((N + 16 * t.rt - 1) / (16 * t.rt));
     const double wb = t.rt * 32.0 * t.ks, xb = t.tt * 32.0 * t.ks;  // bytes of a stage
-    const double stage_w = wb / 25e3, stage_all = (wb + xb) / (t.ns > 2 ? 46e3 : 36e3);
+    const double stage_w = wb / 25e3, stage_all = (wb + xb) / 46e3;
     const double stage = stage_w > stage_all ? stage_w : stage_all;  // us
     for (int s = 1; s <= 8; ++s) {
       if (s > 1 && ((long long)s * M > kMaxTokenSplits || tiles >= 2LL * ncu)) break;

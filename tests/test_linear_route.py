@@ -86,3 +86,18 @@ def test_reported_workspace_serves_tensors_on_and_off_the_bounds(tmp_path):
     CHECK(lin::route(M, N, K, 256, b[0], b[1], b[2], b[3], b[4], on).tiled.splits == s[3]);
     CHECK(lin::route(M, N, K, 256, b[0] + 8, b[1], b[2], b[3], b[4], any).splits == s[4]);
   }""")
+
+
+def test_oracle_shapes_reach_every_tile(tmp_path):
+    """The shapes that the GPU tests hold to the oracle run every tile of the plan, unsplit and split."""
+    from tests.test_gpu_bf16_tiled import EVERY_TILE
+    shapes = ", ".join("{%d, %d, %d, %d, %d}" % s for s in EVERY_TILE)
+    run_rules(tmp_path, "const int shapes[][5] = {" + shapes + r"""};
+  bool seen[bt::kNumTiles][2] = {};
+  for (auto& s : shapes) {
+    const bt::Plan p = lin::tiled_plan(s[0], s[1], s[2], 256);
+    CHECK(p.ok && p.tile == s[3] && p.splits == s[4]);
+    CHECK(s[1] % (16 * bt::kTiles[p.tile].rt) != 0 && s[0] % 16 != 0);
+    seen[p.tile][p.splits > 1] = true;
+  }
+  for (auto& t : seen) CHECK(t[0] && t[1]);""")

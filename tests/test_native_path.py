@@ -104,12 +104,35 @@ def _dense(ops):
     return out
 
 
+class _Recorder:
+    """The native functions, with the names of those that took a call (and those that left one) noted."""
+
+    def __init__(self, nat):
+        self.nat, self.took, self.left = nat, set(), set()
+
+    def __getattr__(self, name):
+        def call(*args):
+            r = getattr(self.nat, name)(*args)
+            (self.left if r is None else self.took).add(name)
+            return r
+        return call
+
+
+OPERATORS = {
+    "_moe": {"moe_route_topk", "moe_permute", "moe_w13_fp8", "quant_act_e4m3", "moe_w2_fp8", "moe_combine",
+             "moe_w13_w4a16"},
+    "_dense": {"linear_bf16", "fp8_gemm_blockscale", "fp8_gemm_ue8m0"}}
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("calls", [_moe, _dense])
 def test_gives_the_bits_of_the_python_path(hip, monkeypatch, calls):
     from ferret_amd import ops
     print(f"[case] native path {calls.__name__}", flush=True)
+    rec = _Recorder(lib.native())
+    monkeypatch.setattr(lib, "native", lambda: rec)
     here = calls(ops)
+    assert rec.took == OPERATORS[calls.__name__] and not rec.left
     monkeypatch.setattr(lib, "native", lambda: lib._Absent())
     there = calls(ops)
     torch.cuda.synchronize()

@@ -2,6 +2,18 @@
 from tests.test_linear_route import run_rules
 
 
+def kernel(tmp_path, M, N, K, workspace=True):
+    """The kernel and K splits of a call with all the workspace it can use, or with none: ("small", splits) for the
+    small-tile kernel, ("128x128", splits) and ("256x128", 1) for the tiled one."""
+    out = run_rules(tmp_path, f"const int M = {M}, N = {N}, K = {K}, mb = (M + 127) / 128, t256 = (N + 255) / 256 * mb;"
+                              f"const f8::Route r = f8::route(M, N, K, false, {'f8::workspace(M, N, K)' if workspace else 0});"
+                              r"""
+  const bool half = r.splits > 1 || (2 * t256 <= f8::kRound && N / 128 * mb <= f8::kRound);
+  std::printf("%s %d", r.mid.ok ? "small" : half ? "128x128" : "256x128", r.mid.ok ? r.mid.splits : r.splits);""",
+                    "fp8_plan.hpp").split()
+    return out[0], int(out[1])
+
+
 def test_each_kernel_asks_for_its_own_partials(tmp_path):
     """A workspace of the 128 x 128 tiles' split keeps that split where the small tiles' is larger, with either
     matrix instruction, and the UE8M0 entry takes it."""
@@ -41,3 +53,14 @@ def test_small_tiles_take_one_round(tmp_path):
   for (auto& s : taken) CHECK(f8::mid_plan(s[0], s[1], s[2]).ok);
   const int left[][3] = {{23, 34944, 1024}, {24, 36608, 5376}, {20, 10624, 11904}, {172, 5248, 128}, {100, 4096, 7168}};
   for (auto& s : left) CHECK(!f8::mid_plan(s[0], s[1], s[2]).ok);""", "fp8_plan.hpp")
+
+
+def test_oracle_shapes_reach_every_small_tile(tmp_path):
+    """One shape per tile of the small-tile kernel, unsplit and split, of those the GPU tests hold to the oracle."""
+    run_rules(tmp_path, r"""
+  const int shapes[][4] = {{17, 128, 128, 0}, {24, 4096, 7168, 0}, {48, 1152, 128, 1}, {33, 256, 2432, 1}, {33, 8320, 128, 2},
+    {33, 1152, 1664, 2}, {129, 1024, 256, 3}, {65, 128, 3072, 3}, {65, 8320, 256, 4}, {65, 1152, 1408, 4}};
+  for (int i = 0; i < 2 * mid::kNumTiles; ++i) {
+    const mid::Plan p = f8::mid_plan(shapes[i][0], shapes[i][1], shapes[i][2]);
+    CHECK(p.ok && p.tile == i / 2 && shapes[i][3] == i / 2 && (p.splits > 1) == (i % 2 == 1));
+  }""", "fp8_plan.hpp")

@@ -18,7 +18,7 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K", [
     (17, 128, 128), (32, 4096, 384), (33, 256, 2432), (48, 1152, 128), (64, 7168, 640), (65, 128, 3072), (24, 4096, 7168),
     (96, 384, 1152), (100, 2048, 4224), (128, 4096, 512), (129, 1024, 256), (200, 640, 1664), (256, 256, 3072),
-    (31, 7168, 16384),
+    (31, 7168, 16384), (33, 8320, 128), (33, 1152, 1664), (65, 8320, 256), (65, 1152, 1408),
     # past 256 tokens, never split: every tile, odd block counts, the last shape of one round and the first past it
     (257, 1024, 128), (300, 256, 2432), (1313, 128, 384), (490, 1024, 1152), (512, 2048, 640), (1024, 2048, 512),
     (1025, 2048, 512), (269, 1536, 16384)])

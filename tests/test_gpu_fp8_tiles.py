@@ -22,6 +22,7 @@ import torch
 from oracle import gemm as G
 from oracle import metrics as MT
 from tests.gpu_helpers import assert_gemm_close, bf16_out, codes8, f32, moe_sample_pairs
+from tests.test_fp8_route import kernel
 
 pytestmark = pytest.mark.gpu
 
@@ -64,11 +65,12 @@ def test_square_kernel_shapes(hip, ops, M, N, K):
     assert torch.equal(y.view(torch.int16), y2.view(torch.int16)), "non-deterministic output"
 
 
-@pytest.mark.parametrize("path", ["square", "tiled"])
-def test_zero_scale_blocks(ops, path):
+@pytest.mark.parametrize("path", ["square", "tiled", "small"])
+def test_zero_scale_blocks(ops, tmp_path, path):
     """A zero activation or weight block scale removes that block's products,
     whatever the e4m3 bytes hold (the oracle multiplies them by 0)."""
-    M, N, K = (3000, 4096, 512) if path == "square" else (700, 512, 512)
+    M, N, K = {"square": (3000, 4096, 512), "tiled": (1100, 2048, 512), "small": (700, 512, 512)}[path]
+    assert path == "square" or kernel(tmp_path, M, N, K)[0] == ("small" if path == "small" else "128x128")
     _say(f"zero-scale blocks, {path} path M={M} N={N} K={K}")
     a, sa, b, sb = _inputs(M, N, K, 80)
     sa[5:9, 1] = 0.0         # four tokens, K block 1

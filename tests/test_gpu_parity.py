@@ -19,6 +19,7 @@ from oracle import metrics as MT
 
 from tests.gpu_helpers import (assert_gemm_close, bf16_out, bits16, codes8, f32, moe_sample_pairs,
                                oracle_routing)
+from tests.test_fp8_route import kernel
 
 pytestmark = pytest.mark.gpu
 
@@ -213,14 +214,18 @@ def test_fp8_gemm_small(ops, M, N, K):
     assert_gemm_close(bf16_out(c), ref, f"fp8 M={M}")
 
 
-@pytest.mark.parametrize("M,N,K", [(128, 256, 1024), (77, 1024, 2048), (256, 512, 1024)])
-def test_fp8_gemm_workspace_and_plain_paths(hip, ops, M, N, K):
-    """16 < M <= 256: the split-K path (workspace given) and the plain path
-    (ws NULL, or one byte too small) both meet the oracle."""
+@pytest.mark.parametrize("M,N,K,split", [
+    (128, 256, 1024, ("small", 1)), (77, 1024, 2048, ("small", 8)), (256, 512, 1024, ("small", 1)),
+    (256, 512, 7168, ("small", 8)), (100, 4096, 7168, ("128x128", 8)), (200, 2048, 7168, ("128x128", 8))])
+def test_fp8_gemm_workspace_and_plain_paths(hip, ops, tmp_path, M, N, K, split):
+    """16 < M <= 256: the path with a workspace (K split by the kernel named,
+    unless 1) and the plain path (ws NULL, or one byte too small) both meet the
+    oracle."""
+    assert kernel(tmp_path, M, N, K) == split
     _say(f"fp8_gemm workspace/plain M={M} N={N} K={K}")
     a, sa, b, sb = _fp8_inputs(M, N, K, seed=3 * M + K)
     need = ops.fp8_workspace_bytes(M, N, K)
-    assert need >= 2 * M * N * 4, "shape expected to take the split-K path"
+    assert need >= 2 * M * N * 4 and need >= split[1] * M * N * 4, "shape expected to take the split-K path"
     ref = G.fp8_blockscale_gemm(codes8(a), f32(sa), codes8(b), f32(sb))
     ws = torch.empty(need, dtype=torch.uint8, device="cuda")
     for ws_ptr, ws_bytes, tag in ((ws.data_ptr(), need, "split"), (None, 0, "null-ws"),
@@ -233,26 +238,20 @@ def test_fp8_gemm_workspace_and_plain_paths(hip, ops, M, N, K):
         assert_gemm_close(bf16_out(c), ref, f"fp8 {tag} M={M}")
 
 
-def _tile_config(M, N):
-    """The tiled configuration of a shape run without a workspace, by the dispatch
-    rule of ferret_fp8_gemm_tiled: 128 x 128 tiles where the 256 x 128 grid
-    would fill at most half of 256 CUs and the 128 x 128 grid fits them."""
-    mb = -(-M // 128)
-    t256, t128 = -(-N // 256) * mb, (N // 128) * mb
-    return "128x128" if 2 * t256 <= 256 and t128 <= 256 else "256x128"
-
-
 @pytest.mark.parametrize("M,N,K,cfg", [
-    (128, 256, 128, "128x128"), (256, 256, 256, "128x128"), (384, 512, 384, "128x128"), (512, 256, 640, "128x128"),
-    (520, 3072, 1536, "128x128"), (1000, 1024, 512, "128x128"),
+    (128, 256, 128, "128x128"), (1152, 2048, 256, "128x128"), (1100, 2048, 384, "128x128"),
+    (1152, 2048, 640, "128x128"), (1000, 3072, 1536, "128x128"), (1100, 2048, 512, "128x128"),
+    (256, 256, 256, "small"), (384, 512, 384, "small"), (512, 256, 640, "small"), (520, 3072, 1536, "small"),
+    (1000, 1024, 512, "small"),
     (1152, 4096, 128, "256x128"), (1152, 4096, 256, "256x128"), (1100, 4096, 384, "256x128"),
     (1100, 4096, 640, "256x128")])
-def test_fp8_gemm_staggered_short_k(hip, M, N, K, cfg):
+def test_fp8_gemm_staggered_short_k(hip, tmp_path, M, N, K, cfg):
     """Without a workspace both tiled configurations run the staggered
     two-half loop; K of 1, 2, 3 and 5 K-steps covers its prologue (three
     stages in flight for one half) and its last-stage waits, on full and
-    partial last token tiles (M % 128 != 0), above M = 256 too."""
-    assert _tile_config(M, N) == cfg
+    partial last token tiles (M % 128 != 0), above M = 256 too.  The smaller
+    shapes of the kind run the small-tile kernel."""
+    assert kernel(tmp_path, M, N, K, workspace=False)[0] == cfg
     _say(f"fp8_gemm staggered M={M} N={N} K={K} ({cfg} tiles)")
     a, sa, b, sb = _fp8_inputs(M, N, K, seed=11 * M + K)
     ref = G.fp8_blockscale_gemm(codes8(a), f32(sa), codes8(b), f32(sb))

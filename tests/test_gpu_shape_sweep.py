@@ -3,8 +3,8 @@ dense and decode-MoE entry points, against the oracle:
 
 - FP8 block-scaled GEMM at M <= 16 (stream-kernel configurations by K-steps
   per wave, the 14-wave single-unit case, the per-unit kernel, N not a
-  multiple of 128), 16 < M <= 256 (split-K tiles with a workspace) and M up to
-  640 (256 x 128 tiles);
+  multiple of 128), 16 < M <= 256 and M up to 640 (small tiles), and larger
+  products (split-K, 128 x 128 and 256 x 128 tiles);
 - bf16 linear at decode M, with and without residual, from a few row units per
   CU to many (the 4-wave units whose first unit interleaves its activations
   with its weight stages, across token-tile and K-split boundaries);
@@ -47,6 +47,8 @@ def _fp8_shapes():
         out.append((int(rng.integers(17, 257)), 128 * int(rng.integers(1, 17)), 128 * int(rng.integers(1, 41))))
     for _ in range(4):  # M up to 640
         out.append((int(rng.integers(257, 641)), 128 * int(rng.integers(1, 9)), 128 * int(rng.integers(1, 25))))
+    # most of the 16 < M draws run the small-tile kernel: these the 128 x 128 tiles, split and not, and the 256 x 128
+    out += [(100, 4096, 6016), (200, 2048, 7168), (1100, 2048, 896), (1100, 4096, 384)]
     return out
 
 

@@ -28,8 +28,8 @@ CHECKER = r"""
 #include "stream_plan.hpp"
 using namespace ferret;
 
-struct Cfg { const char* name; bool silu; int rb; int nw; bool grouped; int max_split; };
-// every try_stream<F, EPI, RB, D, NW> instantiation in skinny.hip
+struct Cfg { const char* name; bool silu; int rb; int nw; bool grouped; int max_split; int per_cu = 1; };
+// every try_stream<F, EPI, RB, D, NW> and try_half_stream<F, EPI, RB, D> instantiation in skinny.hip
 static const Cfg kCfgs[] = {
   {"bf16 linear, 8 waves (+ split-K)", false, 1, 8, false, 8},
   {"bf16 linear, 4 waves", false, 1, 4, false, 1},
@@ -38,6 +38,7 @@ static const Cfg kCfgs[] = {
   {"fp8 dense, 8 waves", false, 1, 8, false, 1},
   {"fp8 moe w13 (SiLU)", true, 2, 8, true, 1},
   {"fp8 moe w2, four blocks per unit", false, 4, 4, true, 1},
+  {"fp8 moe w2, two work-groups of 2 waves per CU", false, 4, 2, true, 1, 2},
   {"int4 moe w13 (SiLU)", true, 2, 8, true, 1},
 };
 
@@ -76,15 +77,16 @@ static void walk(const Cfg& c, int N, int K, int tiles, int ns, int grid, int nt
 
 int main() {
   const int Ns[] = {16, 32, 48, 64, 96, 128, 256, 512, 1024, 2048, 3072, 4096, 6144, 7168, 24576, 153600};
-  const int Ks[] = {128, 256, 384, 512, 896, 1024, 1536, 2048, 3584, 4096, 7168, 8192, 12288, 16384};
+  const int Ks[] = {128, 256, 384, 512, 640, 768, 896, 1024, 1536, 1792, 2048, 3584, 4096, 7168, 8192, 12288, 16384};
   const int Tiles[] = {1, 2, 3, 7, 8, 16, 63, 64, 65, 127, 300, 1000, 4096};
   const int Grids[] = {80, 256, 304};
   for (const Cfg& c : kCfgs)
     for (int N : Ns)
       for (int K : Ks)
         for (int tiles : Tiles)
-          for (int grid : Grids)
+          for (int cus : Grids)
             for (int ns = 1; ns <= c.max_split; ++ns) {
+              const int grid = cus * c.per_cu;
               const StreamPlan p = stream_plan(c.silu, c.rb, c.nw, N, K, tiles, c.grouped, ns, grid);
               if (!p.ok) continue;
               ++plans;
@@ -132,22 +134,27 @@ def test_walker_rejects_the_rb_mismatch_that_faulted(tmp_path):
 
 
 def _instantiations():
-    """(silu, RB, NW, grouped) of every try_stream<F, EPI, RB, D[, NW]>(a, dense_tiles, max_tiles, st)
-    call in skinny.hip (NW defaults to 8; a call with dense_tiles 0 is grouped)."""
+    """(silu, RB, NW, grouped, work-groups per CU) of every try_stream<F, EPI, RB, D[, NW]>(a, dense_tiles,
+    max_tiles, st) call in skinny.hip (NW defaults to 8; a call with dense_tiles 0 is grouped), and of every
+    try_half_stream<F, EPI, RB, D>(a, max_tiles, st) (2 waves, two work-groups per CU, grouped)."""
     import re
     src = open(os.path.join(CSRC, "skinny.hip")).read()
     pat = re.compile(r"try_stream<\s*(\w+)\s*,\s*(\w+)\s*,\s*(\d+)\s*,\s*(\d+)\s*(?:,\s*(\d+)\s*)?>\s*"
                      r"\(\s*a\s*,\s*([^,]+?)\s*,\s*([^,]+?)\s*,\s*st\s*\)")
-    calls = [(m.group(2) == "kSilu", int(m.group(3)), int(m.group(5) or 8), m.group(6) == "0")
+    half = re.compile(r"try_half_stream<\s*(\w+)\s*,\s*(\w+)\s*,\s*(\d+)\s*,\s*(\d+)\s*>\s*\(\s*a\s*,")
+    calls = [(m.group(2) == "kSilu", int(m.group(3)), int(m.group(5) or 8), m.group(6) == "0", 1)
              for m in pat.finditer(src)]
-    return calls, src.count("try_stream<")   # the template's definition is `try_stream(`
+    calls += [(m.group(2) == "kSilu", int(m.group(3)), 2, True, 2) for m in half.finditer(src)]
+    # the templates' definitions are `try_stream(` and `try_half_stream(`
+    return calls, src.count("try_stream<") + src.count("try_half_stream<")
 
 
 def _walker_cfgs():
     import re
     body = CHECKER[CHECKER.index("kCfgs[] = {"):CHECKER.index("};", CHECKER.index("kCfgs[] = {"))]
-    return {(m.group(1) == "true", int(m.group(2)), int(m.group(3)), m.group(4) == "true")
-            for m in re.finditer(r'\{"[^"]*",\s*(true|false),\s*(\d+),\s*(\d+),\s*(true|false),\s*\d+\}', body)}
+    return {(m.group(1) == "true", int(m.group(2)), int(m.group(3)), m.group(4) == "true", int(m.group(5) or 1))
+            for m in re.finditer(r'\{"[^"]*",\s*(true|false),\s*(\d+),\s*(\d+),\s*(true|false),\s*\d+(?:,\s*(\d+))?\}',
+                                 body)}
 
 
 def test_walker_covers_every_try_stream_instantiation():
@@ -155,8 +162,8 @@ def test_walker_covers_every_try_stream_instantiation():
     skinny.hip must appear in it, so an added or changed one cannot escape the
     bounds walk."""
     calls, n_sites = _instantiations()
-    assert len(calls) == n_sites >= 9, (len(calls), n_sites)   # the regex saw every call site
+    assert len(calls) == n_sites >= 10, (len(calls), n_sites)   # the regex saw every call site
     cfgs = _walker_cfgs()
-    assert len(cfgs) >= 6   # distinct (silu, RB, NW, grouped) tuples of the eight entries
+    assert len(cfgs) >= 7   # distinct (silu, RB, NW, grouped, per CU) tuples of the nine entries
     missing = sorted(set(calls) - cfgs)
-    assert not missing, f"try_stream instantiations not walked by the plan walk (silu, RB, NW, grouped): {missing}"
+    assert not missing, f"try_stream instantiations not walked by the plan walk (silu, RB, NW, grouped, per CU): {missing}"

@@ -35,6 +35,12 @@ static_assert(kLds <= 80 * 1024, "two work-groups share a CU's LDS");
 // of N = 4096: 188 / 188, 196 / 185, 222 / 187; N = 4096, K = 7168, 384 experts at
 // 13: 1385 / 1434); checkpoint layout, whose half cache lines the shorter ring
 // fetches later, 14: 428 / 464, 16: 495 / 481.
+// From K = 4096 on the checkpoint layout gains less, and items that come out a
+// little over a whole number of rounds (two work-groups per CU) cost more: at least
+// 3 rounds if every expert had one group or by the 32-row groups there must be, and
+// 20 rows per expert, or 2 and 40.  N = 1792, 128 experts at 17 rows 293 / 355, N =
+// 1280, 64 experts at 64 rows 273 / 336, N = 2816, 96 experts at 36 rows 545 / 639;
+// past the line 1.17 times as fast (82 shapes, none slower), below it 1.05 (94).
 // Other K run on the per-unit kernel, a tile and 16 gate rows per work-group and
 // nothing in flight at its ends: N = 2048, K = 5120, 64 experts 2 / 4 / 8 / 16 rows
 // 108 / 120 / 134 / 199 against 82 / 83 / 84 / 91 us; N = 1024, K = 1024, 128
@@ -46,8 +52,12 @@ static_assert(kLds <= 80 * 1024, "two work-groups share a CU's LDS");
 // 4096 reach the line at 96 rows per expert (24 / 64 / 96 / 256 rows: 32 / 73 / 99 /
 // 244 against 46 / 69 / 71 / 167), 48 experts of 512 at 128 (48 / 64 / 128 rows: 79 /
 // 96 / 176 against 80 / 82 / 127).
-inline bool takes(long long num_pairs, int E, int N, int max_tiles, int ncu, bool stream, bool tiled) {
+inline bool takes(long long num_pairs, int E, int N, int nkb, int max_tiles, int ncu, bool stream, bool tiled) {
   const long long least_rows = stream ? (tiled ? 14 : 16) : 4, nb = N / kItemRows;
+  if (stream && !tiled && nkb >= 32) {
+    const long long items = (E > num_pairs / 32 ? E : num_pairs / 32) * nb;
+    if (items < (num_pairs >= 40LL * E ? 4LL : 6LL) * ncu || num_pairs < 20LL * E) return false;
+  }
   return N % kItemRows == 0 && max_tiles <= kMaxTiles && num_pairs >= least_rows * E &&
          (E * nb >= 2LL * ncu || num_pairs / 32 * nb >= ncu + ncu / 2);
 }

@@ -498,7 +498,7 @@ static int moe_w13_w4a16(const void* x, const int32_t* wq, const void* ws, const
   const bool stream = (eighth == 2 || eighth == 4 || eighth == 7 || eighth == 8) && (bits(ws) & 15) == 0;
   const int span = stream ? eighth : unit_steps(nkb);
   if (span != 0 && ((bits(x) | bits(wq)) & 15) == 0 && (bits(ws) & 3) == 0 && (bits(out) & 7) == 0 &&
-      i4::takes((long long)T * topk, E, N, max_tiles, cu_count(), stream, F == kINT4T))
+      i4::takes((long long)T * topk, E, N, nkb, max_tiles, cu_count(), stream, F == kINT4T))
     return ferret_int4_moe(a, F == kINT4T, span, max_tiles, cu_count(), st);
   const int rc = try_stream<F, kSilu, 2, 5, 8>(a, 0, max_tiles, st);
   if (rc != 1) return rc;

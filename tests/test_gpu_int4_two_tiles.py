@@ -13,6 +13,7 @@ import torch
 
 from oracle import gemm as G
 from tests.gpu_helpers import assert_gemm_close, bf16_out, bits16
+from tests.test_linear_route import run_rules
 
 pytestmark = pytest.mark.gpu
 
@@ -34,14 +35,19 @@ def ops(hip):
                                    (600, 256, 2048), (130, 1024, 2048),                  # a long table; the stream kernel's K
                                    (64, 2048, 2432),                                     # ragged last span
                                    (33, 4096, 7168),
-                                   (8, 1024, 2048)])                                     # few experts of many rows
-def test_two_tiles_equal_one(ops, E, N, K):
+                                   (8, 1024, 2048), (8, 2560, 7168)])                    # few experts of many rows
+def test_two_tiles_equal_one(ops, tmp_path, E, N, K):
     rows = _rows(E) if E > 8 else [n * 24 for n in EDGES[:8]]
     P = sum(rows)
     streams = K in (2048, 7168)  # the K of the stream kernel: 14 (tiled) or 16 rows per expert, else 4
     padded = P // (14 if streams else 4) + 1
     print(f"[case] int4 two tiles E={E} P={P} N={N} K={K}", flush=True)
-    assert 16 * E <= P and padded <= 1024 and (E * (N // 256) >= 512 or P // 32 * (N // 256) >= 384)
+    assert padded <= 1024
+    # tiled weights, then the checkpoint layout, whose line lies higher for the stream kernel's larger K
+    for is_tiled, taken in ((1, 1), (0, (E, K) != (33, 7168))):
+        run_rules(tmp_path, f"CHECK(i4::takes({P}, {E}, {N}, {K // 128}, 4096, 256, {int(streams)}, {is_tiled}) == {int(taken)});"
+                            f"CHECK(!i4::takes({P}, {padded}, {N}, {K // 128}, 4096, 256, {int(streams)}, {is_tiled}));",
+                  "int4_moe.hpp")
     ids = np.concatenate([np.full(n, e, dtype=np.int32) for e, n in enumerate(rows)])
     np.random.default_rng(E).shuffle(ids)
     ids = torch.from_numpy(ids.reshape(-1, 1)).cuda()

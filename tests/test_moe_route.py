@@ -26,3 +26,15 @@ def test_two_tiles_per_unit_only_where_the_units_fill_the_cus(tmp_path):
     {362, 16, 1024, 8, 0}, {432, 16, 896, 28, 0}, {360, 32, 1152, 16, 0}, {6400, 256, 7168, 8, 1}, {4000, 256, 7168, 12, 1},
     {4000, 256, 7168, 6, 1}, {4000, 256, 7168, 14, 1}};
   for (auto& s : w2) CHECK(moe::w2_pairs(s[0], s[1], s[2], s[3], 256) == (s[4] != 0));""", "moe_plan.hpp")
+
+
+def test_int4_checkpoint_layout_asks_for_whole_rounds_at_large_k(tmp_path):
+    run_rules(tmp_path, r"""
+  // num_pairs, E, N, K / 128, taken with the checkpoint layout (the tiled one takes them all)
+  const int shapes[][5] = {{2128, 128, 1792, 56, 0}, {4096, 64, 1280, 56, 0}, {3456, 96, 2816, 56, 0}, {1984, 64, 2304, 56, 0},
+    {7084, 128, 768, 32, 0}, {6400, 128, 4096, 56, 1}, {8192, 128, 1024, 56, 1}, {4096, 384, 4096, 56, 0},
+    {2128, 128, 1792, 16, 1}};
+  for (auto& s : shapes) {
+    CHECK(i4::takes(s[0], s[1], s[2], s[3], 4096, 256, true, false) == (s[4] != 0));
+    CHECK(s[0] < 14 * s[1] || i4::takes(s[0], s[1], s[2], s[3], 4096, 256, true, true));
+  }""", "int4_moe.hpp")

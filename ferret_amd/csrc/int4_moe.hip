@@ -3,7 +3,7 @@
 //
 // The stream kernel takes one tile per unit, so an expert with 17 rows reads
 // and widens its weights twice; next to the bytes of the weights it is the
-// widening (int4 -> bf16 x scale, 20 VALU operations per 8 weights) that bounds
+// widening (int4 -> bf16 x scale, 17 VALU operations per 8 weights) that bounds
 // these products.  Here an item is up to 32 tokens of an expert by 128 gate and
 // 128 up rows over all of K: each widened fragment feeds both tiles' MFMAs, the
 // tokens of a stage are shared by the work-group through LDS, and there is no

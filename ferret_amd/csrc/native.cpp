@@ -4,7 +4,7 @@
 // A decode-sized kernel takes 5 - 15 us; the checks, torch.empty calls and the
 // ctypes call in Python took about 15 us per operator, so a step made of such
 // calls ran at the host's pace (an FP8 projection of 8 tokens: 5.6 us of kernel,
-// 15 us a call).  Here an operator costs about 4 us.
+// 15 us a call).  Here an operator costs about 5 us (a linear of one token 4.6).
 //
 // Every function takes the operator's tensors (None where optional) and returns
 // its result, or None whenever anything is not the plain case: an argument that

@@ -421,8 +421,11 @@ extern "C" int ferret_moe_max_tiles(int num_pairs, int E, int tile_m) {
 }
 
 extern "C" int ferret_moe_tile_m(int num_pairs, int E) {
-  // decode-sized segments (<= ~16 rows per expert) stream weights with the
-  // 16-token skinny kernel; larger segments use 128-row MFMA tiles.
+  // Few rows per expert stream weights with the 16-row tiles of the decode
+  // kernels, more go to 128-row MFMA tiles.  Measured w13 + w2 of 256 experts, 16 /
+  // 128-row tiles (us): even routing, 24 rows 1924 / 2031, 28 rows 2259 / 2068, 32
+  // rows 2706 / 2091; a Zipf(1.1) one is faster on 128 from 12 rows on (16: 2256 /
+  // 1944), which the average does not show.
   return (E > 0 && num_pairs / E >= 32) ? 128 : 16;
 }
 

@@ -2,9 +2,10 @@
 // on gfx950: the HBM-bound bf16 / FP8 / INT4 linear projections and MoE w13
 // grouped GEMMs.
 //
-// Work decomposition.  A unit is (token tile, RB blocks of 16 weight rows); a
-// work-group of NW waves owns a contiguous range of units (a persistent grid
-// of one work-group per CU), and within a unit wave w takes the K-steps
+// Work decomposition.  A unit is (token tile, RB blocks of 16 weight rows), or
+// with TB = 2 (grouped FP8) up to two tiles of an expert; a work-group of NW
+// waves owns a contiguous range of units (a persistent grid of one work-group
+// per CU, two of the 2-wave ones), and within a unit wave w takes the K-steps
 // [w*KS, (w+1)*KS) (one K-step = 128 K = one fp32 scale block), so the unit's
 // partial sums meet once, in LDS, at the end of the unit.
 //

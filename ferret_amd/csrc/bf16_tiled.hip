@@ -19,8 +19,8 @@
 // plan, G at a time, and sums them itself, in the order and from the K rotation
 // of the plan's own tiles: their results bit for bit with no partials in memory.
 // For the allocation-free entry where the 16-token kernels need no split, so that
-// calls there share no memory.  Over 1468 such shapes of 1 .. 128 tokens 1.43
-// times as fast as those kernels (geometric mean; 43 of them more than 4 % slower,
+// calls there share no memory.  Over 1509 such shapes of 1 .. 128 tokens 1.44
+// times as fast as those kernels (geometric mean; 32 of them more than 4 % slower,
 // by up to 33 %), the split form about 1.7 times.
 //
 // Measured, start to now (the 16-token stream kernel once per 16 tokens):

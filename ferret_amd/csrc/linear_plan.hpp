@@ -52,13 +52,18 @@ inline int stream_splits(int M, int N, int K, int ncu) {
 //     16-token tiles x N x K the line lies at 2^25 against the stream kernel (4
 //     tiles of 2048 x 2048, 2^24: 9.7 against 7.0 us; 2 of 4096 x 4096, 2^25:
 //     10.4 against 13.9) and at 10 * 2^20 against the per-unit one (2 tiles of
-//     4096 x 640: 5.8 against 5.3; 4: 6.7 against 7.7).
+//     4096 x 640: 5.8 against 5.3; 4: 6.7 against 7.7).  Up to 3 tokens a
+//     split of a K below 3584 asks for 12 * 2^20: 6352 x 1664 at one token 10.2
+//     against 7.3, 4256 x 2688 11.0 against 9.5; and up to 16 the 128-token tile is
+//     not split below K = 2048 (6464 x 1664 at 4 10.3 against 7.7).
 inline bt::Plan tiled_plan(int M, int N, int K, int ncu) {
   const bool stream = stream_plan(false, 1, 8, N, K, 1, false, stream_splits(M, N, K, ncu), ncu).ok ||
                       (N / 16 >= 4 * ncu && stream_plan(false, 1, 4, N, K, 1, false, 1, ncu).ok);
   const long long work = (long long)((M + 15) / 16) * N * K;
   if ((stream && M <= 16) || work < (stream ? 32LL : 10LL) << 20) return bt::Plan{};
-  return bt::plan(M, N, K, ncu);
+  const bt::Plan p = bt::plan(M, N, K, ncu);
+  const bool few = (M <= 3 && K < 3584 && work < 12LL << 20) || (M <= 16 && K < 2048 && bt::kTiles[p.tile].tt == 8);
+  return p.splits > 1 && few ? bt::Plan{} : p;
 }
 
 // The tiled kernel copies x and the weights global -> LDS 16 bytes at a time,

@@ -101,3 +101,12 @@ def test_oracle_shapes_reach_every_tile(tmp_path):
     seen[p.tile][p.splits > 1] = true;
   }
   for (auto& t : seen) CHECK(t[0] && t[1]);""")
+
+
+def test_few_tokens_split_a_short_k_only_from_a_larger_product_on(tmp_path):
+    run_rules(tmp_path, r"""
+  const int left[][3] = {{1, 6352, 1664}, {1, 4256, 2688}, {3, 7056, 1536}, {2, 3760, 2944}, {1, 3168, 3328},
+    {4, 6464, 1664}, {7, 6288, 1792}};
+  for (auto& s : left) CHECK(!lin::tiled_plan(s[0], s[1], s[2], 256).ok);
+  const int taken[][3] = {{4, 6352, 2560}, {16, 4400, 2432}, {13, 6032, 1920}, {1, 1536, 9984}, {1, 9200, 1152}, {1, 8016, 1664}, {3, 5232, 2432}};
+  for (auto& s : taken) CHECK(lin::tiled_plan(s[0], s[1], s[2], 256).ok);""")
